@@ -648,9 +648,13 @@ extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
     const int gm = flash_gate_mode("mb_flash_ema_bwd", flags, N, hd);
     if (gm < 0) return gm;
     if (gm == 2) {
-        // hi + lo tiles of both kinds and both W fragment sets in LDS: one slot per batch
+        // hi + lo tiles of both kinds and both W fragment sets in LDS: one slot per batch at
+        // head_dim 64, two (N > 32) or four at head_dim 32, whose W fragments and rows take half:
+        // a batch's barrier, loads and stores are shared by its slots, and a slot of 32 dims is
+        // too short to cover them (B3 T201 H6 N33: backward 449 us with one slot per batch, 356 us
+        // with two).
         if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, st) : launch_bwd<64, 2, 1, true, true>(a, vr, st);
-        return NS == 1 ? launch_bwd<32, 1, 1, true, true>(a, vr, st) : launch_bwd<32, 2, 1, true, true>(a, vr, st);
+        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, st) : launch_bwd<32, 2, 2, true, true>(a, vr, st);
     }
     if (gm == 1) {  // the gate's lo tile and W_lo beside the hi ones
         if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, st) : launch_bwd<64, 2, 2, true>(a, vr, st);
