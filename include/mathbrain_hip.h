@@ -223,6 +223,37 @@ int mb_flash_ema_fwd(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, i
 int64_t mb_flash_ema_fwd_workspace(int B, int H, int L, int hd, int K, int N, int flags);
 
 /*
+ * Slot lists: for every 32-step block of every sequence, the valid slots that can be nonzero
+ * in it (a nonzero chunk-start state, or an occurrence before the block's last step).  A slot
+ * left out has zero counters at all the block's steps: gate, score and value are 0, it adds
+ * e^0 to the softmax sum and nothing to any gradient, so mb_flash_ema_fwd_lists and
+ * mb_flash_ema_bwd_lists walk the lists and count the rest.  (A slot's E_k / E_v rows are not
+ * read in the blocks that leave it out: a non-finite value in them reaches the other blocks
+ * only.)  No counterpart in the reference.
+ *
+ *   slot_lists  mb_flash_ema_slot_lists_bytes(B, L, K) bytes of device memory, 16-byte aligned;
+ *               written from x, unique and C_bounds (arguments as mb_flash_ema_fwd) and valid
+ *               for calls with the same ones
+ */
+int64_t mb_flash_ema_slot_lists_bytes(int B, int L, int K);
+int mb_flash_ema_slot_lists(const int64_t *x, int64_t x_sb, int64_t x_sl, const int64_t *unique,
+                            const float *C_bounds, int B, int L, int K, int N, int Np, int nc,
+                            int Br, void *slot_lists, void *stream);
+
+/*
+ * mb_flash_ema_fwd over slot lists (NULL: mb_flash_ema_fwd).  With `scores`, the entries of the
+ * pairs that the lists leave out (all of them 0) are not written; mb_flash_ema_bwd_lists with
+ * the same lists does not read them.
+ */
+int mb_flash_ema_fwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t q_sd,
+                           const int64_t *x, int64_t x_sb, int64_t x_sl, const float *E_k,
+                           const float *E_v, const float *W_pe, const float *rhos,
+                           const int64_t *unique, const float *C_bounds, int B, int H, int L,
+                           int hd, int K, int N, int Np, int nc, int Br, int64_t V_total,
+                           int flags, float *O, float *LSE, float *scores, void *workspace,
+                           int64_t workspace_bytes, const void *slot_lists, void *stream);
+
+/*
  * Flash-EMA gated cross-attention backward.  Replaces FlashEMAFunction.backward and its
  * kernels _flash_ema_bwd_dq_de / _flash_ema_bwd_dw (mathbrain/triton_flash_ema.py:586-650,
  * :250-355, :359-469) with one fused pass.  Arguments as mb_flash_ema_fwd, plus
@@ -259,6 +290,16 @@ int mb_flash_ema_bwd(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, i
                      const float *LSE, int B, int H, int L, int hd, int K, int N, int Np, int nc,
                      int Br, int64_t V_total, int flags, const float *scores, float *dQ,
                      float *dE_k, float *dE_v, float *dW_pe, void *stream);
+
+/* mb_flash_ema_bwd over slot lists (NULL: mb_flash_ema_bwd); see mb_flash_ema_slot_lists. */
+int mb_flash_ema_bwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t q_sd,
+                           const float *dO, const int64_t *x, int64_t x_sb, int64_t x_sl,
+                           const float *E_k, const float *E_v, const float *W_pe,
+                           const float *rhos, const int64_t *unique, const float *C_bounds,
+                           const float *O, const float *LSE, int B, int H, int L, int hd, int K,
+                           int N, int Np, int nc, int Br, int64_t V_total, int flags,
+                           const float *scores, float *dQ, float *dE_k, float *dE_v, float *dW_pe,
+                           const void *slot_lists, void *stream);
 
 /*
  * Flash-EMA attention forward with the query gating folded into its prologue.  Replaces

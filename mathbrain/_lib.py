@@ -36,10 +36,17 @@ SIGNATURES = {
     "mb_unique_rows": ([_p, _i64, _i64, _i, _i, _p, _i, _p, _p], _i),
     "mb_flash_ema_fwd": ([_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _p,
                           _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p, _p, _i64, _p], _i),
+    "mb_flash_ema_fwd_lists": ([_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _p,
+                                _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p, _p, _i64, _p, _p], _i),
+    "mb_flash_ema_slot_lists": ([_p, _i64, _i64, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p], _i),
+    "mb_flash_ema_slot_lists_bytes": ([_i, _i, _i], _i64),
     "mb_flash_ema_fwd_workspace": ([_i, _i, _i, _i, _i, _i, _i], _i64),
     "mb_flash_ema_bwd": ([_p, _i64, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _p, _p,
                           _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p, _p,
                           _p, _p], _i),
+    "mb_flash_ema_bwd_lists": ([_p, _i64, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _p, _p,
+                                _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p, _p,
+                                _p, _p, _p], _i),
     "mb_flash_ema_fwd_gq": ([_p, _i64, _i64, _p, _i64, _i64, _p, _p, _f, _p, _p, _i64, _i64, _p, _p, _p,
                              _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p], _i),
     "mb_gating_fwd": ([_p, _i64, _p, _i64, _p, _p, _i64, _p, _i, _p, _p, _i64, _i, _i, _f, _p, _p,

@@ -81,10 +81,10 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
 
     const int D = a.H * HDR;
     const int ntb = (a.L + kTB - 1) / kTB;
-    const int logical = xcd_major(blockIdx.x, gridDim.x);
-    const int hg = logical % a.head_groups;
-    const int b = logical / (a.head_groups * ntb);
-    const int t0 = ((logical / a.head_groups) % ntb) * kTB;
+    const FlashBlock blk = flash_block(blockIdx.x, a.B, ntb, a.head_groups);
+    const int hg = blk.r;
+    const int t0 = blk.t * kTB;
+    const int b = blk.b;
     const int cbi = t0 / a.Br;
     const int cb = cbi * a.Br;
 
@@ -183,6 +183,8 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
     flash_setup<NPAD>(a, b, t0, cb, win, powt, kinfo);
     const int kend = kinfo[1];
     const int nb = (kend + SB - 1) / SB;
+    const int bi0 = 0;
+    const int bi1 = nb;
 
     // Per-lane rows: steps t = t0 + 16 th + 4 g + i, dims d = 16 dt + c16 of head h.
     const float qscale = 1.0f / sqrtf((float)HDR);
@@ -217,6 +219,7 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         for (int nt = 0; nt < NTW; ++nt) dWacc[dt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     Producer<NPAD, SB, MAXI, MAXE> prod;
+    MetaFeed<SB> feed;
     const int col0 = hg * hpg * HD;  // WID columns from here are staged (zeros past D)
     // Forward scores of a batch, one float per thread (SCN <= blockDim.x): one register held
     // across the slot loop, not four.  The thread's (head, step) is the same in every batch,
@@ -231,15 +234,14 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         const int hs = SUB ? hg * (hpg >> 1) + (hh >> 1) : hg * hpg + hh;
         if (t < a.L && hh < hpg) lse2s = a.LSEin[((int64_t)b * a.H + hs) * a.L + t] * kLog2e;
     }
-    auto load_scores = [&](int batch) {
+    auto load_scores = [&](const BatchMeta* bm) {
         if (!HAS_S || (int)threadIdx.x >= SCN) return;
         const int j = threadIdx.x / (kBwdHeads * kTB);
         const int hh = (threadIdx.x / kTB) % kBwdHeads;
         const int t = t0 + threadIdx.x % kTB;
-        const int k = batch * SB + j;
         const int hs = SUB ? hg * (hpg >> 1) + (hh >> 1) : hg * hpg + hh;  // the scores' head
-        s2pre = (k < kend && t < a.L && hh < hpg)
-                    ? a.S2in[(((int64_t)b * a.H + hs) * a.K + k) * a.L + t]
+        s2pre = (bm[j].row >= 0 && t < a.L && hh < hpg)
+                    ? a.S2in[(((int64_t)b * a.H + hs) * a.K + bm[j].k) * a.L + t]
                     : 0.f;
     };
     auto store_scores = [&](float* dst) {
@@ -249,34 +251,38 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
     auto wait_e_lds = [&]() {
         if constexpr (MAXE == 0) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     };
-    if (nb > 0) {
-        flash_batch_meta<SB>(a, b, 0, kend, win, meta_of(0));
-        if (VR) __syncthreads();  // the load reads the batch's token ids
-        prod.template load<VR>(a, b, cbi, 0, kend, D, col0, WID, meta_of(0));
-        if constexpr (MAXE == 0) prod.template load_e_lds<VR>(a, b, 0, kend, D, col0, WID, meta_of(0), E_of(0));
-        load_scores(0);
+    if (bi1 > bi0) {
+        feed.fetch(a, b, t0, bi0, kend);
+        feed.put(a, b, bi0, kend, win, meta_of(bi0));
+        if (bi0 + 1 < bi1) feed.fetch(a, b, t0, bi0 + 1, kend);
+        __syncthreads();  // the load reads the batch's slots
+        prod.template load<VR>(a, b, cbi, D, col0, WID, meta_of(bi0));
+        if constexpr (MAXE == 0) prod.template load_e_lds<VR>(a, b, D, col0, WID, meta_of(bi0), E_of(0));
+        load_scores(meta_of(bi0));
         __syncthreads();
         store_scores(S2_of(0));
-        prod.template store<TT, S::CROW, S::TROW, PG, PW, S::CDEC, S::CT>(t0, cb, powt, meta_of(0), cdec_of(0), cdecT_of(0), E_of(0), WID,
+        prod.template store<TT, S::CROW, S::TROW, PG, PW, S::CDEC, S::CT>(t0, cb, powt, meta_of(bi0), cdec_of(0), cdecT_of(0), E_of(0), WID,
                                                                      ctile);
-        if (nb > 1) flash_batch_meta<SB>(a, b, 1, kend, win, meta_of(1));
+        if (bi0 + 1 < bi1) feed.put(a, b, bi0 + 1, kend, win, meta_of(bi0 + 1));
         wait_e_lds();
         __syncthreads();
     }
 
-    for (int bi = 0; bi < nb; ++bi) {
-        const int cur = bi & 1;
-        if (bi + 1 < nb) {
-            prod.template load<VR>(a, b, cbi, bi + 1, kend, D, col0, WID, meta_of(bi + 1));
+    for (int bi = bi0; bi < bi1; ++bi) {
+        const int cur = (bi - bi0) & 1;
+        if (bi + 2 < bi1) feed.fetch(a, b, t0, bi + 2, kend);
+        if (bi + 1 < bi1) {
+            prod.template load<VR>(a, b, cbi, D, col0, WID, meta_of(bi + 1));
             if constexpr (MAXE == 0)
-                prod.template load_e_lds<VR>(a, b, bi + 1, kend, D, col0, WID, meta_of(bi + 1), E_of(cur ^ 1));
-            load_scores(bi + 1);
+                prod.template load_e_lds<VR>(a, b, D, col0, WID, meta_of(bi + 1), E_of(cur ^ 1));
+            load_scores(meta_of(bi + 1));
         }
         const _Float16* cdec = cdec_of(cur);
         const float* E = E_of(cur);
         const BatchMeta* meta = meta_of(bi);
         for (int j = 0; j < SB; ++j) {
-            if (meta[j].u < 0) continue;  // padding slot (uniform across the workgroup)
+            const BatchMeta slot = meta[j];
+            if (slot.row < 0) continue;  // padding slot (uniform across the workgroup)
             if (!active) {                // a wave without a head: only the exchange barriers
                 if (SUB) {
                     float unused[4] = {0.f, 0.f, 0.f, 0.f};
@@ -433,8 +439,7 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
             // dE: this lane's 4 steps summed in registers; the 4 row groups (other steps)
             // are reduce-scattered with v_permlane16/32_swap so that row g holds dim tile g
             // (DT = 4) or rows 0 and 2 hold tiles 0 and 1 (DT = 2); one atomic per lane.
-            const int64_t slot_row = VR ? min(meta[j].u, e_rows_of(a) - 1) : (int64_t)b * a.K + bi * SB + j;
-            const int64_t erow = slot_row * D + col0 + hl * HD;
+            const int64_t erow = e_row<VR>(a, b, slot) * D + col0 + hl * HD;
             if (DT == 4) {
                 const float vk = rows4_reduce_scatter(dEk[0], dEk[1 % DT], dEk[2 % DT], dEk[3 % DT]);
                 const float vv = rows4_reduce_scatter(dEv[0], dEv[1 % DT], dEv[2 % DT], dEv[3 % DT]);
@@ -501,11 +506,11 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
                 }
             }
         }
-        if (bi + 1 < nb) {
+        if (bi + 1 < bi1) {
             prod.template store<TT, S::CROW, S::TROW, PG, PW, S::CDEC, S::CT>(t0, cb, powt, meta_of(bi + 1), cdec_of(cur ^ 1), cdecT_of(cur ^ 1),
                                                 E_of(cur ^ 1), WID, ctile);
             store_scores(S2_of(cur ^ 1));
-            if (bi + 2 < nb) flash_batch_meta<SB>(a, b, bi + 2, kend, win, meta_of(bi + 2));
+            if (bi + 2 < bi1) feed.put(a, b, bi + 2, kend, win, meta_of(bi + 2));
         }
         wait_e_lds();
         __syncthreads();
@@ -599,19 +604,21 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, hipStream_t st) {
 }
 
 int flash_validate(const char* who, const FlashArgs& a, int hd);
+void flash_use_lists(FlashArgs& a, const void* lists);
 
 }  // namespace mb
 
 using namespace mb;
 
-extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
-                                int64_t q_sd, const float* dO, const int64_t* x, int64_t x_sb,
-                                int64_t x_sl, const float* E_k, const float* E_v,
-                                const float* W_pe, const float* rhos, const int64_t* unique,
-                                const float* C_bounds, const float* O, const float* LSE, int B,
-                                int H, int L, int hd, int K, int N, int Np, int nc, int Br,
-                                int64_t V_total, int flags, const float* scores, float* dQ,
-                                float* dE_k, float* dE_v, float* dW_pe, void* stream) {
+extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                                      int64_t q_sd, const float* dO, const int64_t* x, int64_t x_sb,
+                                      int64_t x_sl, const float* E_k, const float* E_v,
+                                      const float* W_pe, const float* rhos, const int64_t* unique,
+                                      const float* C_bounds, const float* O, const float* LSE, int B,
+                                      int H, int L, int hd, int K, int N, int Np, int nc, int Br,
+                                      int64_t V_total, int flags, const float* scores, float* dQ,
+                                      float* dE_k, float* dE_v, float* dW_pe, const void* slot_lists,
+                                      void* stream) {
     FlashArgsV a{};
     a.Q = Q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sl = q_sl; a.q_sd = q_sd;
     a.dO = dO; a.x = x; a.x_sb = x_sb; a.x_sl = x_sl;
@@ -622,10 +629,12 @@ extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
     a.silu = (flags & MB_FLASH_SILU) ? 1 : 0;
     a.dQ = dQ; a.dEk = dE_k; a.dEv = dE_v; a.dW = dW_pe;
     a.S2in = scores;
+    flash_use_lists(a, slot_lists);
     const bool vr = (flags & MB_FLASH_VOCAB_ROWS) != 0;
     a.e_rows = vr ? V_total : 0;
     int rc = flash_validate("mb_flash_ema_bwd", a, hd);
     if (rc) return rc;
+    MB_REQUIRE(((uintptr_t)slot_lists & 15) == 0, "mb_flash_ema_bwd: slot_lists must be 16-byte aligned");
     MB_REQUIRE(!vr || V_total >= 1, "mb_flash_ema_bwd: MB_FLASH_VOCAB_ROWS needs V_total >= 1 rows");
     // dE_k, dE_v and dW_pe are accumulated with atomics, so they are cleared first -- also
     // when there is no step to accumulate (B or L zero), which leaves them zero; every dQ
@@ -673,4 +682,17 @@ extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
     if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, st);
     if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, st);
     return launch_bwd<32, 4, 2>(a, vr, st);
+}
+
+extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                                int64_t q_sd, const float* dO, const int64_t* x, int64_t x_sb,
+                                int64_t x_sl, const float* E_k, const float* E_v,
+                                const float* W_pe, const float* rhos, const int64_t* unique,
+                                const float* C_bounds, const float* O, const float* LSE, int B,
+                                int H, int L, int hd, int K, int N, int Np, int nc, int Br,
+                                int64_t V_total, int flags, const float* scores, float* dQ,
+                                float* dE_k, float* dE_v, float* dW_pe, void* stream) {
+    return mb_flash_ema_bwd_lists(Q, q_sb, q_sh, q_sl, q_sd, dO, x, x_sb, x_sl, E_k, E_v, W_pe, rhos, unique,
+                                  C_bounds, O, LSE, B, H, L, hd, K, N, Np, nc, Br, V_total, flags, scores, dQ,
+                                  dE_k, dE_v, dW_pe, nullptr, stream);
 }

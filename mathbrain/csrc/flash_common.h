@@ -1,7 +1,7 @@
 // Pieces shared by the flash-EMA forward and backward kernels (gfx950).
 //
-// Both kernels work on one (sequence b, 32-step block) per workgroup and walk the valid
-// slots of b in batches of SB.  For every batch the whole workgroup first builds, in LDS,
+// Both kernels work on one (sequence b, 32-step block) per workgroup and walk the block's
+// slots (its list, flash_slots.hip, or all valid slots of b) in batches of SB.  For every batch the whole workgroup first builds, in LDS,
 //   cdec[j][t][n]  (fp16)  the decayed key-side counter c_dec[t, u_j, n] that gates step t,
 //   cdecT[j][n][t] (bf16)  the same counter, transposed, for the backward's dW_pe product,
 //   E[j][0|1][D]   (fp32)  the slot's key and value embeddings,
@@ -47,6 +47,21 @@ constexpr int kTB = 32;      // time steps per workgroup
 constexpr int kMaxWin = 64;  // positions [cb, t0 + 32) of the match window
 constexpr float kCMax = 65504.0f - kMaxWin;  // chunk-start counters saturate here (fp16)
 
+// One slot as the slot loops take it: its index in the sequence's list (`k`, the row of
+// C_bounds, of the scores and of gathered E rows), its row of a vocabulary table (`row`, the
+// token id; negative: a padding slot, which nothing reads) and its occurrences in the match
+// window (bit p: x[cb + p] is the slot's token).
+struct __align__(16) BatchMeta {
+    uint64_t mask;
+    int32_t row;
+    int32_t k;
+};
+
+// Slots of one 32-step block that can be nonzero in it, and the sequence's valid slots.
+struct SlotCount {
+    int32_t active, valid;
+};
+
 struct FlashArgs {
     const float* Q;
     int64_t q_sb, q_sh, q_sl, q_sd;
@@ -73,7 +88,11 @@ struct FlashArgs {
     float* dEk;  // like Ek, accumulated with atomics (zeroed by the host)
     float* dEv;
     float* dW;   // [N, D], accumulated with atomics (zeroed by the host)
-    int head_groups;  // backward: workgroups per (b, block) along heads
+    int head_groups;  // workgroups per (b, block) along heads
+    // NULL, or the blocks' slot lists of mb_flash_ema_slot_lists: [B, ntb, K] entries and
+    // [B, ntb] counts; a workgroup then walks its block's list instead of all K slots
+    const BatchMeta* list;
+    const SlotCount* nlist;
 };
 
 // Arguments of the kernels whose E_k / E_v (and dE_k / dE_v) rows are token ids into
@@ -179,12 +198,21 @@ __device__ inline float row_sum16(float v) {
     return v;
 }
 
-// Workgroup id -> logical id so that consecutive logical ids (the blocks of one
-// sequence, which share its slot embeddings) land on the same XCD and its L2:
-// the dispatcher hands workgroups to the 8 XCDs round-robin.
-__device__ inline int xcd_major(int bid, int G) {
-    if (G % 8) return bid;
-    return (bid % 8) * (G / 8) + bid / 8;
+// Workgroup id -> (sequence b, 32-step block t, index r < inner within them), the blocks from
+// the last to the first: a block's slot list grows with the steps before it, and the longest
+// workgroups first leave the shortest for the end, when the rounds run out of step (at B56 T512
+// the first-to-last order cost 0.8 of the forward's 11.2 ms: an eighth workgroup on a CU whose
+// others took seven).  With B a multiple of 8 each XCD keeps its own sequences (the dispatcher
+// hands workgroups to the 8 XCDs round-robin), whose slot embeddings then share its L2.
+struct FlashBlock {
+    int b, t, r;
+};
+__device__ inline FlashBlock flash_block(int bid, int B, int ntb, int inner) {
+    const int xcds = B % 8 ? 1 : 8;
+    const int per = B / xcds;
+    const int l = bid / xcds;
+    const int q = l / inner;
+    return FlashBlock{bid % xcds * per + q % per, ntb - 1 - q / per, l % inner};
 }
 
 // LDS carve-up of the per-batch staging buffers: cdec (fp16), with BF the transposed bf16
@@ -226,23 +254,21 @@ static inline int flash_gate_mode(const char* who, int flags, int N, int hd) {
     return N <= 64 && hd <= 64 ? 1 : 0;
 }
 
-// Row of slot (b, k), token id u, in E_k / E_v / dE_k / dE_v: b*K + k, or with VR
-// the token id (padding slots, -1, read row 0; ids are clamped to the table).  u comes from
-// the batch's slot info in LDS: a global read here would make the producer's other loads
-// wait with it (memory reads complete in order).
+// Row of a slot in E_k / E_v / dE_k / dE_v: b*K + k, or with VR the token id (clamped to
+// the table).  The slot comes from the batch's slot info in LDS: a global read here would
+// make the producer's other loads wait with it (memory reads complete in order).
 template <bool VR, class A>
-__device__ inline int64_t e_row(const A& a, int b, int k, int64_t u) {
-    if (!VR) return (int64_t)b * a.K + k;
-    return min(max(u, (int64_t)0), e_rows_of(a) - 1);
+__device__ inline int64_t e_row(const A& a, int b, const BatchMeta& m) {
+    if (!VR) return (int64_t)b * a.K + m.k;  // (b * K is uniform)
+    return min((int64_t)max(m.row, 0), e_rows_of(a) - 1);
 }
 
-struct BatchMeta {
-    int64_t u;
-    uint64_t mask;
-};
+// Token id as BatchMeta holds it: ids past 2^31 - 1 clamp (e_row clamps to the table anyway).
+__device__ inline int32_t slot_row(int64_t u) { return (int32_t)min(u, (int64_t)INT32_MAX); }
 
 // Per-workgroup setup shared by both kernels: the match window tokens, the rho^j table
-// (j = 0..64) and the valid-slot range of sequence b.
+// (j = 0..64), kinfo[0] = the valid slots of sequence b and kinfo[1] = the slots to walk (the
+// length of the block's list, or without lists one past the last valid slot).
 template <int NPAD>
 __device__ void flash_setup(const FlashArgs& a, int b, int t0, int cb, int64_t* win,
                             float* powt, int* kinfo) {
@@ -269,6 +295,15 @@ __device__ void flash_setup(const FlashArgs& a, int b, int t0, int cb, int64_t* 
         kinfo[1] = 0;   // one past the last valid slot
     }
     __syncthreads();
+    if (a.list) {  // (uniform)
+        const SlotCount n = a.nlist[(int64_t)b * ((a.L + kTB - 1) / kTB) + t0 / kTB];
+        if (tid == 0) {
+            kinfo[0] = n.valid;
+            kinfo[1] = n.active;
+        }
+        __syncthreads();
+        return;
+    }
     int cnt = 0, last = 0;
     for (int k = tid; k < a.K; k += nthr) {
         if (a.unique[(int64_t)b * a.K + k] >= 0) {
@@ -297,24 +332,44 @@ __device__ inline int split_tiles(const FlashArgs& a, int lane) {
     return 32.0f * b0 < fmaxf(b0, b1) ? 2 : 3;
 }
 
-// Slot ids and 64-bit occurrence masks of batch `bi`: wave j < SB handles slot j.
+// Slot info of the batches, on its way into the LDS ring.  From a block's list: the first
+// 4 SB lanes of wave 0 read one word each of a batch's entries (`fetch`, before the loads of
+// the batch before it, whose wait then covers this one) and write them to the ring at that
+// batch's end (`put`).  Read where they are written, the entries would be waited for behind the
+// slots' atomics and score stores (vector-memory waits count in order); scalar loads made
+// wave 0's LDS waits wait for them too (fp32 mode at head_dim 32: backward 470 against 449 us).
+// Without lists (`put` alone) wave j < SB looks up slot bi * SB + j and its occurrence mask.
 template <int SB>
-__device__ void flash_batch_meta(const FlashArgs& a, int b, int bi, int kend, const int64_t* win,
-                                 BatchMeta* meta) {
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int nwaves = blockDim.x >> 6;
-    for (int j = wave; j < SB; j += nwaves) {
-        const int k = bi * SB + j;
-        const int64_t u = (k < kend) ? a.unique[(int64_t)b * a.K + k] : (int64_t)-1;
-        const bool hit = u >= 0 && win[lane] == u;
-        const uint64_t m = __ballot(hit);
-        if (lane == 0) {
-            meta[j].u = u;
-            meta[j].mask = m;
+struct MetaFeed {
+    static_assert(SB * sizeof(BatchMeta) <= 256, "one word per lane");
+    uint32_t word;
+
+    // entries of batch bi (of a list of kend)
+    __device__ void fetch(const FlashArgs& a, int b, int t0, int bi, int kend) {
+        if (!a.list || threadIdx.x >= 4 * SB) return;
+        const int64_t blk = (int64_t)b * ((a.L + kTB - 1) / kTB) + t0 / kTB;
+        const int i = bi * SB + (int)threadIdx.x / 4;
+        word = reinterpret_cast<const uint32_t*>(a.list + blk * a.K + min(i, kend - 1))[threadIdx.x % 4];
+        if (i >= kend && threadIdx.x % 4 == 2) word = 0xFFFFFFFFu;  // row = -1: past the list
+    }
+
+    __device__ void put(const FlashArgs& a, int b, int bi, int kend, const int64_t* win, BatchMeta* meta) const {
+        if (a.list) {  // (uniform)
+            if (threadIdx.x < 4 * SB) reinterpret_cast<uint32_t*>(meta)[threadIdx.x] = word;
+            return;
+        }
+        const int wave = threadIdx.x >> 6;
+        const int lane = threadIdx.x & 63;
+        const int nwaves = blockDim.x >> 6;
+        for (int j = wave; j < SB; j += nwaves) {
+            const int k = bi * SB + j;
+            const int64_t u = (k < kend) ? a.unique[(int64_t)b * a.K + k] : (int64_t)-1;
+            const bool hit = u >= 0 && win[lane] == u;
+            const uint64_t m = __ballot(hit);
+            if (lane == 0) meta[j] = BatchMeta{m, u < 0 ? -1 : slot_row(u), k};
         }
     }
-}
+};
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -330,11 +385,11 @@ struct Producer {
     // The batch's E_k / E_v rows ([SB][2][width] floats) into E with global_load_lds_dwordx4:
     // wave w issues the 1 KB pieces w, w + waves, ...; lane l of a piece moves float4 64 c + l,
     // which lands at E + 4 (64 c + l) (the instruction writes lane l's 16 bytes at the LDS
-    // address in M0 plus 16 l).  Rows of slots past kend are not loaded (no slot reads them).
+    // address in M0 plus 16 l).  Rows of padding slots are not loaded (nothing reads them).
     // The caller waits for the loads (vmcnt) before the barrier that publishes E.
     template <bool VR, class A>
-    __device__ void load_e_lds(const A& a, int b, int bi, int kend, int D, int col0, int width,
-                               const BatchMeta* meta, float* E) const {
+    __device__ void load_e_lds(const A& a, int b, int D, int col0, int width, const BatchMeta* meta,
+                               float* E) const {
         const int w4 = width / 4;
         const int nvec = SB * 2 * w4;
         const int lane = threadIdx.x & 63;
@@ -345,18 +400,15 @@ struct Producer {
             const int r = i % (2 * w4);
             const int which = r / w4;
             const int c4 = r % w4;
-            const int k = bi * SB + j;
-            if (i < nvec && k < kend && col0 + c4 * 4 < D) {
-                const float* src =
-                    (which ? a.Ev : a.Ek) + e_row<VR>(a, b, k, VR ? meta[j].u : 0) * D + col0 + c4 * 4;
+            if (i < nvec && meta[j].row >= 0 && col0 + c4 * 4 < D) {
+                const float* src = (which ? a.Ev : a.Ek) + e_row<VR>(a, b, meta[j]) * D + col0 + c4 * 4;
                 __builtin_amdgcn_global_load_lds(src, (lds_void*)(E + 256 * c), 16, 0, 0);
             }
         }
     }
 
     template <bool VR, class A>
-    __device__ void load(const A& a, int b, int cbi, int bi, int kend, int D, int col0,
-                         int width, const BatchMeta* meta) {
+    __device__ void load(const A& a, int b, int cbi, int D, int col0, int width, const BatchMeta* meta) {
         const int tid = threadIdx.x;
         const int nthr = blockDim.x;
 #pragma unroll
@@ -364,10 +416,10 @@ struct Producer {
             const int item = tid + ii * nthr;
             const int j = item / BPS;
             const int n0 = (item % (NPAD / 4)) * 4;
-            const int k = bi * SB + j;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (j < SB && k < kend) {
-                const float* src = a.Cb + (((int64_t)b * a.nc + cbi) * a.K + k) * a.Np + n0;
+            if (j < SB && meta[j].row >= 0) {
+                const float* src = a.Cb + ((int64_t)b * a.nc + cbi) * a.K * a.Np + n0 +
+                                   (uint64_t)(uint32_t)meta[j].k * (uint32_t)a.Np;
                 if (n0 + 3 < a.N && (a.Np & 3) == 0) {
                     v = *reinterpret_cast<const float4*>(src);
                 } else {
@@ -390,11 +442,9 @@ struct Producer {
                 const int r = i % (2 * w4);
                 const int which = r / w4;
                 const int c4 = r % w4;
-                const int k = bi * SB + j;
                 // columns past D (heads a partial head group does not have) stay zero
-                if (k < kend && col0 + c4 * 4 < D) {
-                    const float* src =
-                        (which ? a.Ev : a.Ek) + e_row<VR>(a, b, k, VR ? meta[j].u : 0) * D + col0 + c4 * 4;
+                if (meta[j].row >= 0 && col0 + c4 * 4 < D) {
+                    const float* src = (which ? a.Ev : a.Ek) + e_row<VR>(a, b, meta[j]) * D + col0 + c4 * 4;
                     v = *reinterpret_cast<const float4*>(src);
                 }
             }

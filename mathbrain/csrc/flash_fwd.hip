@@ -22,6 +22,8 @@ int flash_validate(const char* who, const FlashArgs& a, int hd) {
     return MB_OK;
 }
 
+void flash_use_lists(FlashArgs& a, const void* lists);
+
 }  // namespace mb
 
 using namespace mb;
@@ -71,13 +73,14 @@ extern "C" int64_t mb_flash_ema_fwd_workspace(int B, int H, int L, int hd, int K
     return need;
 }
 
-extern "C" int mb_flash_ema_fwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
-                                int64_t q_sd, const int64_t* x, int64_t x_sb, int64_t x_sl,
-                                const float* E_k, const float* E_v, const float* W_pe,
-                                const float* rhos, const int64_t* unique, const float* C_bounds,
-                                int B, int H, int L, int hd, int K, int N, int Np, int nc, int Br,
-                                int64_t V_total, int flags, float* O, float* LSE, float* scores,
-                                void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int mb_flash_ema_fwd_lists(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                                      int64_t q_sd, const int64_t* x, int64_t x_sb, int64_t x_sl,
+                                      const float* E_k, const float* E_v, const float* W_pe,
+                                      const float* rhos, const int64_t* unique, const float* C_bounds,
+                                      int B, int H, int L, int hd, int K, int N, int Np, int nc, int Br,
+                                      int64_t V_total, int flags, float* O, float* LSE, float* scores,
+                                      void* workspace, int64_t workspace_bytes, const void* slot_lists,
+                                      void* stream) {
     FlashArgsV a{};
     a.Q = Q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sl = q_sl; a.q_sd = q_sd;
     a.x = x; a.x_sb = x_sb; a.x_sl = x_sl;
@@ -87,6 +90,7 @@ extern "C" int mb_flash_ema_fwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
     a.silu = (flags & MB_FLASH_SILU) ? 1 : 0;
     a.O = O; a.LSE = LSE;
     a.S2out = scores;
+    flash_use_lists(a, slot_lists);
     const bool vr = (flags & MB_FLASH_VOCAB_ROWS) != 0;
     a.e_rows = vr ? V_total : 0;
     int rc = flash_validate("mb_flash_ema_fwd", a, hd);
@@ -94,9 +98,22 @@ extern "C" int mb_flash_ema_fwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
     MB_REQUIRE(!vr || V_total >= 1, "mb_flash_ema_fwd: MB_FLASH_VOCAB_ROWS needs V_total >= 1 rows");
     MB_REQUIRE(workspace_bytes >= 0, "mb_flash_ema_fwd: negative workspace size %lld", (long long)workspace_bytes);
     MB_REQUIRE(((uintptr_t)workspace & 15) == 0, "mb_flash_ema_fwd: workspace must be 16-byte aligned");
+    MB_REQUIRE(((uintptr_t)slot_lists & 15) == 0, "mb_flash_ema_fwd: slot_lists must be 16-byte aligned");
     if (B == 0 || L == 0) return MB_OK;
     MB_REQUIRE(Q && x && rhos && unique && O && LSE && W_pe, "mb_flash_ema_fwd: null pointer");
     MB_REQUIRE(K == 0 || (E_k && E_v && C_bounds), "mb_flash_ema_fwd: null slot pointer");
     return fwd_dispatch(a, hd, N, flags, vr, (hipStream_t)stream, static_cast<float*>(workspace),
                         workspace ? workspace_bytes : 0, nullptr);
+}
+
+extern "C" int mb_flash_ema_fwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
+                                int64_t q_sd, const int64_t* x, int64_t x_sb, int64_t x_sl,
+                                const float* E_k, const float* E_v, const float* W_pe,
+                                const float* rhos, const int64_t* unique, const float* C_bounds,
+                                int B, int H, int L, int hd, int K, int N, int Np, int nc, int Br,
+                                int64_t V_total, int flags, float* O, float* LSE, float* scores,
+                                void* workspace, int64_t workspace_bytes, void* stream) {
+    return mb_flash_ema_fwd_lists(Q, q_sb, q_sh, q_sl, q_sd, x, x_sb, x_sl, E_k, E_v, W_pe, rhos, unique, C_bounds,
+                                  B, H, L, hd, K, N, Np, nc, Br, V_total, flags, O, LSE, scores, workspace,
+                                  workspace_bytes, nullptr, stream);
 }

@@ -70,14 +70,13 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
 
     const int D = a.H * HD;
     const int ntb = (a.L + kTB - 1) / kTB;
-    const int logical = xcd_major(blockIdx.x, gridDim.x);
-    // one workgroup per (b, slot part, 32-step block, head group); a group holds hpg heads
-    // (hpg divides H), one wave each, and waves past hpg only help stage and synchronise.
-    // The blocks of one (b, part) are neighbours, so they share an XCD's L2 for their rows.
-    const int hg = logical % a.head_groups;
-    const int t0 = ((logical / a.head_groups) % ntb) * kTB;
-    const int part = (logical / (a.head_groups * ntb)) % sp.ksplit;
-    const int b = logical / (a.head_groups * ntb * sp.ksplit);
+    // one workgroup per (b, 32-step block, slot part, head group); a group holds hpg heads
+    // (hpg divides H), one wave each, and waves past hpg only help stage and synchronise
+    const FlashBlock blk = flash_block(blockIdx.x, a.B, ntb, sp.ksplit * a.head_groups);
+    const int hg = blk.r % a.head_groups;
+    const int part = blk.r / a.head_groups;
+    const int t0 = blk.t * kTB;
+    const int b = blk.b;
     const int cbi = t0 / a.Br;
     const int cb = cbi * a.Br;
     const int hpg = a.H / a.head_groups;
@@ -180,8 +179,11 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
     const float qscale = 1.0f / sqrtf((float)HD);
     f32x4 o[TW][DT];
     float m[TW], l[TW];
-    // the absent slots' mass (score 0, no value) joins part 0's softmax sum
-    const float absent = a.v_total >= 0.f && part == 0 ? fmaxf(a.v_total - (float)kvalid, 0.f) : 0.f;
+    // The absent slots' mass (score 0, no value) joins part 0's softmax sum, and so do the
+    // valid slots that the block's list leaves out: their counters are zero at every step of
+    // the block, so their gates, scores and values are.
+    const int skipped = part == 0 && a.list ? kvalid - kend : 0;
+    const float absent = (a.v_total >= 0.f && part == 0 ? fmaxf(a.v_total - (float)kvalid, 0.f) : 0.f) + (float)skipped;
 #pragma unroll
     for (int tt = 0; tt < TW; ++tt) {
         const int t = t0 + 16 * (tile0 + tt) + c16;
@@ -199,40 +201,45 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
                 o[tt][dt][i] = 0.f;
             }
         }
-        m[tt] = a.v_total >= 0.f ? 0.f : -INFINITY;
+        m[tt] = a.v_total >= 0.f || skipped > 0 ? 0.f : -INFINITY;
         l[tt] = absent;
     }
 
     Producer<NPAD, SB, MAXI, MAXE> prod;
+    MetaFeed<SB> feed;
     // MAXE = 0: the rows go to LDS directly; wait for them before the barrier that publishes them
     auto wait_e_lds = [&]() {
         if constexpr (MAXE == 0) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     };
     if (bi1 > bi0) {
-        flash_batch_meta<SB>(a, b, bi0, kend, win, meta_of(bi0));
-        if (VR) __syncthreads();  // the load reads the batch's token ids
-        prod.template load<VR>(a, b, cbi, bi0, kend, D, col0, WIDF, meta_of(bi0));
-        if constexpr (MAXE == 0) prod.template load_e_lds<VR>(a, b, bi0, kend, D, col0, WIDF, meta_of(bi0), E_of(0));
+        feed.fetch(a, b, t0, bi0, kend);
+        feed.put(a, b, bi0, kend, win, meta_of(bi0));
+        if (bi0 + 1 < bi1) feed.fetch(a, b, t0, bi0 + 1, kend);
+        __syncthreads();  // the load reads the batch's slots
+        prod.template load<VR>(a, b, cbi, D, col0, WIDF, meta_of(bi0));
+        if constexpr (MAXE == 0) prod.template load_e_lds<VR>(a, b, D, col0, WIDF, meta_of(bi0), E_of(0));
         __syncthreads();
         prod.template store<false, S::CROW, S::TROW, PREC, false, S::CDEC>(t0, cb, powt, meta_of(bi0), cdec_of(0), nullptr, E_of(0), WIDF, CM);
-        if (bi0 + 1 < bi1) flash_batch_meta<SB>(a, b, bi0 + 1, kend, win, meta_of(bi0 + 1));
+        if (bi0 + 1 < bi1) feed.put(a, b, bi0 + 1, kend, win, meta_of(bi0 + 1));
         wait_e_lds();
         __syncthreads();
     }
 
     for (int bi = bi0; bi < bi1; ++bi) {
         const int cur = (bi - bi0) & 1;
+        if (bi + 2 < bi1) feed.fetch(a, b, t0, bi + 2, kend);
         if (bi + 1 < bi1) {
-            prod.template load<VR>(a, b, cbi, bi + 1, kend, D, col0, WIDF, meta_of(bi + 1));
+            prod.template load<VR>(a, b, cbi, D, col0, WIDF, meta_of(bi + 1));
             if constexpr (MAXE == 0)
-                prod.template load_e_lds<VR>(a, b, bi + 1, kend, D, col0, WIDF, meta_of(bi + 1), E_of(cur ^ 1));
+                prod.template load_e_lds<VR>(a, b, D, col0, WIDF, meta_of(bi + 1), E_of(cur ^ 1));
         }
         const _Float16* cdec = cdec_of(cur);
         const float* E = E_of(cur);
         const BatchMeta* meta = meta_of(bi);
         for (int j = 0; j < SB; ++j) {
             // padding slot (uniform across the workgroup), or a wave without a head
-            if (meta[j].u < 0 || !active) continue;
+            const BatchMeta slot = meta[j];
+            if (slot.row < 0 || !active) continue;
             f16x8 cf[TW][NS];
 #pragma unroll
             for (int tt = 0; tt < TW; ++tt)
@@ -336,7 +343,7 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
                 }
             }
             if (a.S2out && g == 0) {
-                float* srow = a.S2out + (((int64_t)b * a.H + h) * a.K + bi * SB + j) * a.L;
+                float* srow = a.S2out + (((int64_t)b * a.H + h) * a.K + slot.k) * a.L;
 #pragma unroll
                 for (int tt = 0; tt < TW; ++tt) {
                     const int t = t0 + 16 * (tile0 + tt) + c16;
@@ -347,7 +354,7 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
         if (bi + 1 < bi1) {
             prod.template store<false, S::CROW, S::TROW, PREC, false, S::CDEC>(t0, cb, powt, meta_of(bi + 1), cdec_of(cur ^ 1), nullptr,
                                               E_of(cur ^ 1), WIDF, CM);
-            if (bi + 2 < bi1) flash_batch_meta<SB>(a, b, bi + 2, kend, win, meta_of(bi + 2));
+            if (bi + 2 < bi1) feed.put(a, b, bi + 2, kend, win, meta_of(bi + 2));
         }
         wait_e_lds();
         __syncthreads();

@@ -210,8 +210,29 @@ def _slot_rows(E, B, K, D, V_total, what):
     return Ef.contiguous(), False
 
 
+# Blocks x slots below which a call walks every slot instead of listing the active ones: the
+# lists cost a launch of 10 to 30 us, and a call this small spends no more than that on the
+# slots they leave out (B3 T201 N33 in fp32 mode, about 9 000: 577 us without, 616 us with; B8
+# T512, 96 000: 17.6 ms for a 2-layer model's step either way; above that the lists win).
+MIN_LISTED_SLOTS = 16384
+
+
+def _slot_lists(xl, uniq, Cb, N, Br):
+    """The blocks' slot lists of mb_flash_ema_slot_lists (None for a call too small for them)."""
+    B, L = xl.shape
+    K = uniq.shape[1]
+    if B * -(-L // 32) * K < MIN_LISTED_SLOTS:
+        return None
+    nbytes = _lib.lib().mb_flash_ema_slot_lists_bytes(B, L, K)
+    lists = torch.empty(nbytes, dtype=torch.uint8, device=xl.device)
+    _lib.call("mb_flash_ema_slot_lists", _lib.ptr(xl), xl.stride(0), xl.stride(1), _lib.ptr(uniq),
+              _lib.ptr(Cb), B, L, K, N, Cb.shape[3], Cb.shape[1], int(Br), _lib.ptr(lists),
+              _lib.stream(xl.device))
+    return lists
+
+
 def _fwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, V_total, use_silu, Br,
-              absent_mass, return_scores, prec=0):
+              absent_mass, return_scores, prec=0, every_slot=False):
     dev = _lib.require_gpu(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds,
                            what="flash_ema_forward")
     check_counter_range(rhos, "flash_ema_forward")
@@ -241,12 +262,13 @@ def _fwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, V_total, use_
     with torch.cuda.device(dev):
         nws = _fwd_workspace_bytes(B, H, L, hd, K, N, flags, dev.index)
         ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
-        _lib.call("mb_flash_ema_fwd", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(xl), xl.stride(0),
+        lists = None if every_slot else _slot_lists(xl, uniq, Cb, N, Br)
+        _lib.call("mb_flash_ema_fwd_lists", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(xl), xl.stride(0),
                   xl.stride(1), _lib.ptr(Ek), _lib.ptr(Ev), _lib.ptr(W), _lib.ptr(rh),
                   _lib.ptr(uniq), _lib.ptr(Cb), B, H, L, hd, K, N, Cb.shape[3], Cb.shape[1],
                   int(Br), int(V_total), flags, _lib.ptr(O), _lib.ptr(LSE), _lib.ptr(S2), _lib.ptr(ws), nws,
-                  _lib.stream(dev))
-    return O, LSE, S2, Ek, Ev, table
+                  _lib.ptr(lists), _lib.stream(dev))
+    return O, LSE, S2, Ek, Ev, table, lists
 
 
 @functools.lru_cache(maxsize=256)
@@ -315,8 +337,9 @@ def flash_ema_forward(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_
         if Ek.dim() == 2:
             return O, LSE, C_bounds, Ek, Ev
         return O, LSE, C_bounds, Ek.reshape(B, K, H, hd), Ev.reshape(B, K, H, hd)
+    # over every slot, not the blocks' lists: the scores of all (step, slot) pairs are wanted
     res = _forward_with_scores(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_tensor, C_bounds,
-                               use_silu, Br, absent_mass, prec)
+                               use_silu, Br, absent_mass, prec, every_slot=True)[:6]
     # the kernel writes the rows of valid slots only: padding slots' rows hold -inf (score
     # of no slot), as a softmax over them expects
     res[5].masked_fill_((unique_tensor < 0)[:, None, :, None], float("-inf"))
@@ -324,20 +347,22 @@ def flash_ema_forward(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_
 
 
 def _forward_with_scores(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_tensor, C_bounds,
-                         use_silu, Br, absent_mass, prec):
-    """flash_ema_forward's six outputs with the scores [B, H, K_max, L]; the rows of padding
-    slots are left unwritten (the backward never reads them)."""
+                         use_silu, Br, absent_mass, prec, every_slot=False):
+    """flash_ema_forward's six outputs with the scores [B, H, K_max, L], and the slot lists; the
+    scores of padding slots, and of the slots that a block's list leaves out (unless
+    ``every_slot``), are left unwritten (the backward never reads them)."""
     B, H, L, hd = Q.shape
     K = unique_tensor.shape[1]
-    O, LSE, S2, Ek, Ev, table = _fwd_impl(Q, x, E_k_active, E_v_active, W_pe, rhos, unique_tensor,
-                                          C_bounds, V_total, use_silu, Br, absent_mass, True, prec)
+    O, LSE, S2, Ek, Ev, table, lists = _fwd_impl(Q, x, E_k_active, E_v_active, W_pe, rhos, unique_tensor,
+                                                 C_bounds, V_total, use_silu, Br, absent_mass, True, prec,
+                                                 every_slot)
     if table:
-        return O, LSE, C_bounds, Ek, Ev, S2
-    return O, LSE, C_bounds, Ek.view(B, K, H, hd), Ev.view(B, K, H, hd), S2
+        return O, LSE, C_bounds, Ek, Ev, S2, lists
+    return O, LSE, C_bounds, Ek.view(B, K, H, hd), Ev.view(B, K, H, hd), S2, lists
 
 
 def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V_total, use_silu,
-              Br, absent_mass, scores, prec=0):
+              Br, absent_mass, scores, prec=0, lists=None):
     dev = _lib.require_gpu(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO,
                            what="flash_ema_backward")
     check_counter_range(rhos, "flash_ema_backward")
@@ -369,12 +394,14 @@ def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V
                                or not scores.is_contiguous()):
         raise ValueError(f"scores must be contiguous fp32 [B, H, K_max, L], got {tuple(scores.shape)}")
     with torch.cuda.device(dev):
-        _lib.call("mb_flash_ema_bwd", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(dOf), _lib.ptr(xl),
+        if lists is None:
+            lists = _slot_lists(xl, uniq, Cb, N, Br)
+        _lib.call("mb_flash_ema_bwd_lists", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(dOf), _lib.ptr(xl),
                   xl.stride(0), xl.stride(1), _lib.ptr(Ek), _lib.ptr(Ev), _lib.ptr(W),
                   _lib.ptr(rh), _lib.ptr(uniq), _lib.ptr(Cb), _lib.ptr(Of), _lib.ptr(Lf), B, H, L,
                   hd, K, N, Cb.shape[3], Cb.shape[1], int(Br), int(V_total),
                   _flash_flags(use_silu, absent_mass, table, prec), _lib.ptr(scores), _lib.ptr(dQ),
-                  _lib.ptr(dEk), _lib.ptr(dEv), _lib.ptr(dW), _lib.stream(dev))
+                  _lib.ptr(dEk), _lib.ptr(dEv), _lib.ptr(dW), _lib.ptr(lists), _lib.stream(dev))
     return dQ, dEk, dEv, dW
 
 
@@ -516,7 +543,7 @@ class FlashEMAFunction(torch.autograd.Function):
             score_budget.hold(res[5], nbytes)
         O, LSE, C_bounds, E_k, E_v = res[:5]
         ctx.save_for_backward(Q, x, E_k, E_v, W_pe, rhos, C_bounds, unique_tensor, O, LSE,
-                              res[5] if keep else None)
+                              res[5] if keep else None, res[6] if keep else None)
         ctx.V_total = V_total
         ctx.use_silu = use_silu
         ctx.Br = Br
@@ -528,11 +555,15 @@ class FlashEMAFunction(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, dO):
-        Q, x, E_k, E_v, W_pe, rhos, C_bounds, unique_tensor, O, LSE, S2 = ctx.saved_tensors
-        dQ, dEk, dEv, dW = flash_ema_backward(Q, x, E_k, E_v, W_pe, rhos, ctx.V_total,
-                                              unique_tensor, C_bounds, O, LSE, dO.contiguous(),
-                                              ctx.use_silu, ctx.Br, ctx.absent_mass, scores=S2,
-                                              precision=ctx.precision)
+        Q, x, E_k, E_v, W_pe, rhos, C_bounds, unique_tensor, O, LSE, S2, lists = ctx.saved_tensors
+        if S2 is None:
+            dQ, dEk, dEv, dW = flash_ema_backward(Q, x, E_k, E_v, W_pe, rhos, ctx.V_total, unique_tensor,
+                                                  C_bounds, O, LSE, dO.contiguous(), ctx.use_silu, ctx.Br,
+                                                  ctx.absent_mass, precision=ctx.precision)
+        else:
+            dQ, dEk, dEv, dW = _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE,
+                                         dO.contiguous(), ctx.V_total, ctx.use_silu, ctx.Br, ctx.absent_mass,
+                                         S2, _prec(ctx.precision), lists)
         if ctx.W_rows > dW.shape[0]:  # W_pe passed with padded rows: their gradient is 0
             dW = torch.cat([dW, dW.new_zeros(ctx.W_rows - dW.shape[0], dW.shape[1])])
         return dQ, None, dEk, dEv, dW, None, None, None, None, None, None, None, None, None

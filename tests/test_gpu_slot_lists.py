@@ -1,0 +1,98 @@
+"""The blocks' slot lists (mb_flash_ema_slot_lists) against the definition computed on the CPU,
+and the attention over them (mb_flash_ema_fwd_lists / mb_flash_ema_bwd_lists) against the same
+call over every slot: what the lists leave out is exactly zero, so outputs and gradients agree
+to the rounding of reordered fp32 sums (the skipped slots' e^0 terms are added at once, and the
+atomics' order is free): 1e-5 norm-wise.  dW_pe has a bound of its own: its product takes dpre
+in bf16, and a last-bit difference of dpre can round it to the other neighbour, 2^-8 of that
+term and so at most 2^-8 of the sum; in fp32 mode, with its second bf16 part, 2^-16.  The
+default mode's gradients from stored scores are left to the oracle's tests: there a probability
+that rounds to either side of 2^-7 changes a whole slot's gate arithmetic."""
+import pytest
+import torch
+
+from tests.test_gpu_flash import make_case, norm_err
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+TOL_DW = {"fp32": 2.0 ** -16, "bf16": 2.0 ** -8, "fp16": 2.0 ** -8}
+
+
+def lists_of(c, dev):
+    from mathbrain import _lib
+    x, u, Cb = c["x"].to(dev), c["unique"].to(dev), c["Cb"].to(dev).float().contiguous()
+    B, L = x.shape
+    K, N = c["K"], c["rhos"].shape[0]
+    buf = torch.full((_lib.lib().mb_flash_ema_slot_lists_bytes(B, L, K),), 255, dtype=torch.uint8, device=dev)
+    _lib.call("mb_flash_ema_slot_lists", _lib.ptr(x), x.stride(0), x.stride(1), _lib.ptr(u), _lib.ptr(Cb), B, L, K,
+              N, Cb.shape[3], Cb.shape[1], c["Br"], _lib.ptr(buf), _lib.stream(dev))
+    return buf
+
+
+def expected(c):
+    """{(b, block): [k, ...]} of the active slots."""
+    x, u, Cb, Br, N = c["x"], c["unique"], c["Cb"].cpu(), c["Br"], c["rhos"].shape[0]
+    B, L = x.shape
+    out = {}
+    for b in range(B):
+        for blk in range(-(-L // 32)):
+            j = blk * 32 // Br
+            seen = x[b, j * Br:min(blk * 32 + 31, L)]
+            state = (Cb[b, j, :, :N] != 0).any(1)
+            out[b, blk] = [k for k in range(c["K"]) if u[b, k] >= 0 and (state[k] or bool((seen == u[b, k]).any()))]
+    return out
+
+
+def call(c, dev, lists, absent_mass, use_silu, prec):
+    from mathbrain import _lib
+    from mathbrain.triton_flash_ema import _flash_flags, _prec
+    B, H, L, hd = c["Q"].shape
+    K, N, D = c["K"], c["rhos"].shape[0], H * hd
+    cu = lambda t: t.to(dev).float().contiguous()  # noqa: E731
+    Q, Ek, Ev, W, rh, Cb = (cu(c[k]) for k in ("Q", "E_k", "E_v", "W", "rhos", "Cb"))
+    x, u = c["x"].to(dev), c["unique"].to(dev)
+    dO = torch.randn(B, H, L, hd, generator=torch.Generator().manual_seed(3)).to(dev)
+    flags = _flash_flags(use_silu, absent_mass, False, _prec(prec))
+    O, LSE, S2 = (torch.full(s, float("nan"), device=dev) for s in ((B, H, L, hd), (B, H, L), (B, H, K, L)))
+    g = [torch.full(s, float("nan"), device=dev) for s in ((B, H, L, hd), (B, K, D), (B, K, D), (N, D))]
+    p, st = _lib.ptr, _lib.stream(dev)
+    common = (B, H, L, hd, K, N, Cb.shape[3], Cb.shape[1], c["Br"], c["V"], flags)
+    _lib.call("mb_flash_ema_fwd_lists", p(Q), *Q.stride(), p(x), x.stride(0), x.stride(1), p(Ek), p(Ev), p(W), p(rh),
+              p(u), p(Cb), *common, p(O), p(LSE), p(S2), None, 0, p(lists), st)
+    outs = []
+    for scores in (S2, None):
+        _lib.call("mb_flash_ema_bwd_lists", p(Q), *Q.stride(), p(dO), p(x), x.stride(0), x.stride(1), p(Ek), p(Ev),
+                  p(W), p(rh), p(u), p(Cb), p(O), p(LSE), *common, p(scores), *(p(t) for t in g), p(lists), st)
+        outs += [t.cpu() for t in g]
+    return [O.cpu(), LSE.cpu()] + outs
+
+
+@pytest.mark.parametrize("L, N, Br, warmup, pad_slots", [
+    (64, 16, 64, 0, 0),        # no history: the first block sees only its own tokens
+    (97, 33, 64, 40, 5),       # rows that are not float4s, a last block of one step
+    (130, 64, 32, 30, 0),      # a chunk per block
+    (70, 128, 24, 0, 0),       # chunks that do not end where blocks do; single fp16 products
+    (1, 8, 64, 20, 0),         # one step
+    (256, 16, 64, 900, 0),     # more than one round of 512 slots
+])
+@pytest.mark.parametrize("absent_mass", [True, False])
+def test_lists_and_the_attention_over_them(L, N, Br, warmup, pad_slots, absent_mass):
+    dev = torch.device("cuda", 0)
+    c = make_case(2, L, 700, 4, 32, N, warmup=warmup, seed=L + N, qs=0.5, es=0.3, ws=0.2, Br=Br, pad_slots=pad_slots)
+    B, K = c["unique"].shape
+    buf = lists_of(c, dev)
+    nblk = -(-L // 32)
+    entries = buf[:B * nblk * K * 16].view(torch.int32).view(B, nblk, K, 4).cpu()
+    counts = buf[B * nblk * K * 16:].view(torch.int32).view(B, nblk, 2).cpu()
+    for (b, blk), ks in expected(c).items():
+        assert counts[b, blk].tolist() == [len(ks), int((c["unique"][b] >= 0).sum())]
+        assert entries[b, blk, :len(ks), 3].tolist() == ks
+        assert entries[b, blk, :len(ks), 2].tolist() == c["unique"][b, ks].tolist()
+    for use_silu, prec in ((True, "bf16"), (False, "fp32" if N <= 64 else "fp16")):
+        got = call(c, dev, buf, absent_mass, use_silu, prec)
+        want = call(c, dev, None, absent_mass, use_silu, prec)
+        for i, (a, w) in enumerate(zip(got, want)):
+            if prec == "bf16" and 2 <= i <= 5:
+                continue
+            assert torch.isfinite(a).all()
+            assert norm_err(a, w) < (TOL_DW[prec] if i in (5, 9) else TOL)
