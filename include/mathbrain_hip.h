@@ -266,7 +266,8 @@ int mb_flash_ema_fwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q
  *             MB_FLASH_VOCAB_ROWS [V_total, H*hd], the sums over every slot of each token
  *   dW_pe     [N, H*hd] fp32 contiguous output
  *
- * dQ is written once per element.  dE_k, dE_v and dW_pe are cleared by the call (with a
+ * dQ is written once per element, or, where a small grid splits the slots into parts, cleared
+ * and accumulated like the rest.  dE_k, dE_v and dW_pe are cleared by the call (with a
  * fill kernel, no memset) and then accumulated with fp32 atomics, so their summation
  * order is not fixed, as in the reference's tl.atomic_add.  The gate is recomputed as
  * in the forward (the same arithmetic for the same flags), except that by default, when
@@ -291,7 +292,16 @@ int mb_flash_ema_bwd(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, i
                      int Br, int64_t V_total, int flags, const float *scores, float *dQ,
                      float *dE_k, float *dE_v, float *dW_pe, void *stream);
 
-/* mb_flash_ema_bwd over slot lists (NULL: mb_flash_ema_bwd); see mb_flash_ema_slot_lists. */
+/*
+ * mb_flash_ema_bwd over slot lists (NULL: every slot; see mb_flash_ema_slot_lists).
+ *
+ *   workspace  NULL, or workspace_bytes >= mb_flash_ema_bwd_workspace(hd, N) bytes of device
+ *              memory (16-byte aligned, contents irrelevant, one call's at a time): room for
+ *              the workgroups' dW_pe sums where all of them run at once; otherwise, and without
+ *              it, they are added with atomics.  Gradients agree either way up to the order of
+ *              the sums.
+ */
+int64_t mb_flash_ema_bwd_workspace(int hd, int N);
 int mb_flash_ema_bwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t q_sd,
                            const float *dO, const int64_t *x, int64_t x_sb, int64_t x_sl,
                            const float *E_k, const float *E_v, const float *W_pe,
@@ -299,7 +309,8 @@ int mb_flash_ema_bwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q
                            const float *O, const float *LSE, int B, int H, int L, int hd, int K,
                            int N, int Np, int nc, int Br, int64_t V_total, int flags,
                            const float *scores, float *dQ, float *dE_k, float *dE_v, float *dW_pe,
-                           const void *slot_lists, void *stream);
+                           const void *slot_lists, void *workspace, int64_t workspace_bytes,
+                           void *stream);
 
 /*
  * Flash-EMA attention forward with the query gating folded into its prologue.  Replaces

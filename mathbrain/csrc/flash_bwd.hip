@@ -19,7 +19,8 @@
 // across the slot loop, and only the scores s and dp need a sum over the 16 lanes of a
 // DPP row.  Each wave adds its 16 steps' dE_k/dE_v of a slot to global memory with one
 // coalesced atomic per lane (cheaper, measured, than summing the two half-waves in LDS
-// first and flushing once).  dW is added once per wave at the end.
+// first and flushing once).  dW is added once per wave at the end.  Small grids split each
+// workgroup's slots into parts (slot_parts), whose dQ then adds with atomics too.
 #include "flash_common.h"
 
 #include <algorithm>
@@ -34,15 +35,23 @@ constexpr int kMetaRing = 4;
 // probability reaches this at one of the wave's steps (2^-7).
 constexpr float kSplitP = 0.0078125f;
 
-__global__ void zero_fill_kernel(float* p, int64_t n) {
+// Clears up to four arrays in one launch.
+constexpr int kZeroArrays = 4;
+struct ZeroFill {
+    float* p[kZeroArrays];
+    int64_t n[kZeroArrays];
+};
+__global__ void zero_fill_kernel(ZeroFill z) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0.f;
+    for (int k = 0; k < kZeroArrays; ++k)
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < z.n[k]; i += stride) z.p[k][i] = 0.f;
 }
 
-static int zero_fill(float* p, int64_t n, hipStream_t st) {
+static int zero_fill(const ZeroFill& z, hipStream_t st) {
+    const int64_t n = *std::max_element(z.n, z.n + kZeroArrays);
     if (n <= 0) return MB_OK;
     const int blocks = (int)std::min<int64_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(zero_fill_kernel, dim3(blocks), dim3(256), 0, st, p, n);
+    hipLaunchKernelGGL(zero_fill_kernel, dim3(blocks), dim3(256), 0, st, z);
     return check_launch("zero fill");
 }
 
@@ -81,8 +90,9 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
 
     const int D = a.H * HDR;
     const int ntb = (a.L + kTB - 1) / kTB;
-    const FlashBlock blk = flash_block(blockIdx.x, a.B, ntb, a.head_groups);
-    const int hg = blk.r;
+    const FlashBlock blk = flash_block(a, blockIdx.x, ntb, a.ksplit * a.head_groups);
+    const int hg = blk.r % a.head_groups;
+    const int part = blk.r / a.head_groups;  // of the block's slot batches
     const int t0 = blk.t * kTB;
     const int b = blk.b;
     const int cbi = t0 / a.Br;
@@ -180,11 +190,14 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         wfr[f] = v;
         if (PG) wfl[f] = (ctile >> ns) & 1 ? vl : f16x8{};
     }
-    flash_setup<NPAD>(a, b, t0, cb, win, powt, kinfo);
+    flash_powers<NPAD>(a, powt);
+    flash_setup(a, b, t0, cb, win, kinfo);
     const int kend = kinfo[1];
     const int nb = (kend + SB - 1) / SB;
-    const int bi0 = 0;
-    const int bi1 = nb;
+    const int bi0 = part * nb / a.ksplit;  // this part's batches
+    const int bi1 = (part + 1) * nb / a.ksplit;
+    // a part of a short list may have none: it only leaves zeros where its sums are expected
+    if (a.ksplit > 1 && bi0 >= bi1 && !a.dWpart) return;
 
     // Per-lane rows: steps t = t0 + 16 th + 4 g + i, dims d = 16 dt + c16 of head h.
     const float qscale = 1.0f / sqrtf((float)HDR);
@@ -516,7 +529,7 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         __syncthreads();
     }
 
-    // dQ (the gate carried log2 e, the query 1/sqrt(hd)) and dW.
+    // dQ (the gate carried log2 e, the query 1/sqrt(hd)).
     const float qf = kLn2 * qscale;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -524,23 +537,81 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         if (t >= a.L || !active) continue;
         float* dst = a.dQ + (((int64_t)b * a.H + h) * a.L + t) * HDR + sub0;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) dst[16 * dt + c16] = dq[dt][i] * qf;
-    }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int nt = 0; nt < NTW; ++nt) {
-            const int n = 16 * ((XH ? NTW * th : 0) + nt) + c16;
-            if (n >= a.N || !active) continue;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                atomicAdd(&a.dW[(int64_t)n * D + h * HDR + sub0 + 16 * dt + 4 * g + i], dWacc[dt][nt][i]);
+        for (int dt = 0; dt < DT; ++dt) {
+            if (a.ksplit > 1) atomicAdd(dst + 16 * dt + c16, dq[dt][i] * qf);  // the parts' sum, cleared by the host
+            else dst[16 * dt + c16] = dq[dt][i] * qf;
         }
+    }
+    // dW_pe.  The two half-waves of a head hold sums of the same elements (without XH): added
+    // through LDS first (the staging buffers are free after the last batch's barrier).
+    bool mine = active;
+    if (!XH) {
+        f32x4* red = reinterpret_cast<f32x4*>(smem) + hl * DT * NTW * 64 + lane;
+        if (th == 1) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int nt = 0; nt < NTW; ++nt) red[(dt * NTW + nt) * 64] = dWacc[dt][nt];
+        }
+        __syncthreads();
+        if (th == 0) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int nt = 0; nt < NTW; ++nt) dWacc[dt][nt] += red[(dt * NTW + nt) * 64];
+        }
+        mine = mine && th == 0;
+    }
+    if (mine && a.dWpart) {
+        f32x4* dst = reinterpret_cast<f32x4*>(a.dWpart) +
+                     ((int64_t)blockIdx.x * (kBwdHeads * (XH ? 2 : 1)) + hl + (XH ? kBwdHeads * th : 0)) * DT * NTW * 64 + lane;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) dst[(dt * NTW + nt) * 64] = dWacc[dt][nt];
+    } else if (mine) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) {
+                const int n = 16 * ((XH ? NTW * th : 0) + nt) + c16;
+                if (n >= a.N) continue;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    atomicAdd(&a.dW[(int64_t)n * D + h * HDR + sub0 + 16 * dt + 4 * g + i], dWacc[dt][nt][i]);
+            }
+    }
 #undef cdec_of
 #undef cdecT_of
 #undef E_of
 #undef S2_of
 #undef meta_of
+}
+
+// dW_pe [N, D] from the workgroups' sums: one workgroup per 64-lane tile of a head group, its
+// four waves each a quarter of the launch's workgroups of that head group (flash_block's order:
+// workgroup wg takes head group wg % head_groups).
+template <int DT, int NTW, bool XH>
+__global__ void __launch_bounds__(256)
+bwd_dw_kernel(const float* __restrict__ part, int wgs, int head_groups, int cols, int N, int D,
+              float* __restrict__ dW) {
+    constexpr int TILES = kBwdHeads * DT * NTW * (XH ? 2 : 1);
+    __shared__ f32x4 red[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int hg = blockIdx.x / TILES, tile = blockIdx.x % TILES;
+    const f32x4* src = reinterpret_cast<const f32x4*>(part) + tile * 64 + lane;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int wg = wave * head_groups + hg; wg < wgs; wg += 4 * head_groups) v += src[(int64_t)wg * TILES * 64];
+    red[wave][lane] = v;
+    __syncthreads();
+    if (wave) return;
+    v = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+    const int nt = tile % NTW, dt = tile / NTW % DT;
+    const int hl = tile / (NTW * DT) % kBwdHeads, th = tile / (NTW * DT * kBwdHeads);
+    const int n = 16 * (NTW * th + nt) + (lane & 15);
+    const int col = 16 * DT * hl + 16 * dt + 4 * (lane >> 4);  // within the head group's `cols`
+    if (n < N && col < cols) *reinterpret_cast<f32x4*>(dW + (int64_t)n * D + hg * cols + col) = v;
 }
 
 template <int HD, int NS, int SB, bool XH, bool PG, bool PW, bool SUB = false>
@@ -553,7 +624,7 @@ static size_t bwd_lds_bytes() {
 }
 
 template <int HD, int NS, int SB, bool PG = false, bool PW = false, bool SUB = false>
-static int launch_bwd(const FlashArgsV& a0, bool vr, hipStream_t st) {
+static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, hipStream_t st) {
     FlashArgsV a = a0;
     // heads per group: the largest divisor of H that is at most four (with SUB two heads,
     // whose four sub-heads take the four wave pairs)
@@ -572,11 +643,28 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, hipStream_t st) {
     constexpr int NTW = NT < 256 / HD ? NT : 256 / HD;
     constexpr bool XH = NT > NTW;
     static_assert(NT == NTW || NT == 2 * NTW, "at most two half-waves per head");
-    const size_t lds = bwd_lds_bytes<HD, NS, SB, XH, PG, PW, SUB>();
+    const size_t lds = std::max(bwd_lds_bytes<HD, NS, SB, XH, PG, PW, SUB>(),
+                                XH ? (size_t)0 : (size_t)kBwdHeads * (HD / 16) * NTW * 64 * 16);  // dW_pe's halves
     if (lds > 160 * 1024)
         return fail(MB_ERR_UNSUPPORTED, "mb_flash_ema_bwd: hd=%d, N=%d needs %zu B of LDS", HD, a.N, lds);
     const int ntb = (a.L + kTB - 1) / kTB;
-    dim3 grid(a.B * ntb * a.head_groups);
+    // Slot parts (one workgroup per CU: registers).  Their dQ adds with atomics, so it is cleared
+    // with the other sums.  Workgroups that all run at once leave their dW_pe sums in the
+    // workspace, and bwd_dw_kernel adds them up: at the end of such a launch their atomics, on
+    // the same N x D addresses, would come all together (a block of four slots, H8 N64: 36 us,
+    // 22 us with the workspace and the power table's one log2 per rate).
+    const int conc = device_cus();
+    const int64_t G = (int64_t)a.B * ntb * a.head_groups;
+    a.ksplit = slot_parts(G, conc, (a.K + SB - 1) / SB);
+    const int64_t wgs = G * a.ksplit;
+    if (wgs > conc) a.dWpart = nullptr;
+    if (a.ksplit > 1) {
+        zero.p[3] = a.dQ;
+        zero.n[3] = (int64_t)a.B * a.H * a.L * a.hd;
+    }
+    if (a.dWpart) zero.n[0] = 0;  // written whole
+    if (const int rc = zero_fill(zero, st)) return rc;
+    dim3 grid((unsigned)wgs);
 #define MB_BWD_PICK(MI, ME, VR)                                                                  \
     (a.S2in ? (a.silu ? flash_ema_bwd_kernel<HD, NS, SB, MI, ME, true, true, NTW, XH, VR, PG, PW, SUB>       \
                       : flash_ema_bwd_kernel<HD, NS, SB, MI, ME, false, true, NTW, XH, VR, PG, PW, SUB>)     \
@@ -600,6 +688,12 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, hipStream_t st) {
     else return fail(MB_ERR_UNSUPPORTED, "mb_flash_ema_bwd: N=%d too wide", a.N);
 #undef MB_BWD
 #undef MB_BWD_PICK
+    if (a.dWpart) {
+        constexpr int tiles = kBwdHeads * (HD / 16) * NTW * (XH ? 2 : 1);
+        hipLaunchKernelGGL((bwd_dw_kernel<HD / 16, NTW, XH>), dim3(a.head_groups * tiles), dim3(256), 0, st, a.dWpart,
+                           (int)wgs, a.head_groups, (SUB ? 2 : 1) * hpg * HD, a.N, a.H * a.hd,
+                           a.dW);
+    }
     return check_launch("mb_flash_ema_bwd");
 }
 
@@ -610,6 +704,12 @@ void flash_use_lists(FlashArgs& a, const void* lists);
 
 using namespace mb;
 
+extern "C" int64_t mb_flash_ema_bwd_workspace(int hd, int N) {
+    if (hd < 1 || N < 1) return 0;
+    // a workgroup's dW_pe tile: its head group's columns x the rates rounded up to whole tiles
+    return (int64_t)device_cus() * kBwdHeads * std::min(hd, 64) * ((N + 31) / 32 * 32) * 4;
+}
+
 extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
                                       int64_t q_sd, const float* dO, const int64_t* x, int64_t x_sb,
                                       int64_t x_sl, const float* E_k, const float* E_v,
@@ -618,7 +718,7 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
                                       int H, int L, int hd, int K, int N, int Np, int nc, int Br,
                                       int64_t V_total, int flags, const float* scores, float* dQ,
                                       float* dE_k, float* dE_v, float* dW_pe, const void* slot_lists,
-                                      void* stream) {
+                                      void* workspace, int64_t workspace_bytes, void* stream) {
     FlashArgsV a{};
     a.Q = Q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sl = q_sl; a.q_sd = q_sd;
     a.dO = dO; a.x = x; a.x_sb = x_sb; a.x_sl = x_sl;
@@ -630,6 +730,9 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     a.dQ = dQ; a.dEk = dE_k; a.dEv = dE_v; a.dW = dW_pe;
     a.S2in = scores;
     flash_use_lists(a, slot_lists);
+    MB_REQUIRE(workspace_bytes >= 0, "mb_flash_ema_bwd: negative workspace size %lld", (long long)workspace_bytes);
+    MB_REQUIRE(((uintptr_t)workspace & 15) == 0, "mb_flash_ema_bwd: workspace must be 16-byte aligned");
+    if (workspace && workspace_bytes >= mb_flash_ema_bwd_workspace(hd, N)) a.dWpart = static_cast<float*>(workspace);
     const bool vr = (flags & MB_FLASH_VOCAB_ROWS) != 0;
     a.e_rows = vr ? V_total : 0;
     int rc = flash_validate("mb_flash_ema_bwd", a, hd);
@@ -637,19 +740,15 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     MB_REQUIRE(((uintptr_t)slot_lists & 15) == 0, "mb_flash_ema_bwd: slot_lists must be 16-byte aligned");
     MB_REQUIRE(!vr || V_total >= 1, "mb_flash_ema_bwd: MB_FLASH_VOCAB_ROWS needs V_total >= 1 rows");
     // dE_k, dE_v and dW_pe are accumulated with atomics, so they are cleared first -- also
-    // when there is no step to accumulate (B or L zero), which leaves them zero; every dQ
-    // element is written once.
+    // when there is no step to accumulate (B or L zero), which leaves them zero; so is dQ when
+    // the slots are split into parts (else every dQ element is written once).
     const int64_t D = (int64_t)H * hd;
     const int64_t erows = K > 0 ? (vr ? V_total : (int64_t)B * K) : 0;
     MB_REQUIRE(dW_pe, "mb_flash_ema_bwd: null dW_pe");
     MB_REQUIRE(erows == 0 || (dE_k && dE_v), "mb_flash_ema_bwd: null dE_k / dE_v");
     hipStream_t st = (hipStream_t)stream;
-    if ((rc = zero_fill(dW_pe, (int64_t)N * D, st))) return rc;
-    if (erows > 0) {
-        if ((rc = zero_fill(dE_k, erows * D, st))) return rc;
-        if ((rc = zero_fill(dE_v, erows * D, st))) return rc;
-    }
-    if (B == 0 || L == 0) return MB_OK;
+    ZeroFill zero{{dW_pe, dE_k, dE_v}, {(int64_t)N * D, erows * D, erows * D}};
+    if (B == 0 || L == 0) return zero_fill(zero, st);
     MB_REQUIRE(Q && dO && x && rhos && unique && O && LSE && W_pe && dQ,
                "mb_flash_ema_bwd: null pointer");
     MB_REQUIRE(K == 0 || (E_k && E_v && C_bounds), "mb_flash_ema_bwd: null slot pointer");
@@ -662,26 +761,26 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
         // a batch's barrier, loads and stores are shared by its slots, and a slot of 32 dims is
         // too short to cover them (B3 T201 H6 N33: backward 449 us with one slot per batch, 356 us
         // with two).
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, st) : launch_bwd<64, 2, 1, true, true>(a, vr, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, st) : launch_bwd<32, 2, 2, true, true>(a, vr, st);
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, zero, st) : launch_bwd<64, 2, 1, true, true>(a, vr, zero, st);
+        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, zero, st) : launch_bwd<32, 2, 2, true, true>(a, vr, zero, st);
     }
     if (gm == 1) {  // the gate's lo tile and W_lo beside the hi ones
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, st) : launch_bwd<64, 2, 2, true>(a, vr, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, st) : launch_bwd<32, 2, 2, true>(a, vr, st);
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, zero, st) : launch_bwd<64, 2, 2, true>(a, vr, zero, st);
+        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, zero, st) : launch_bwd<32, 2, 2, true>(a, vr, zero, st);
     }
     if (hd == 128) {  // two 64-dim sub-heads per head
-        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, st);
-        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, st);
-        return launch_bwd<64, 4, 1, false, false, true>(a, vr, st);
+        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, zero, st);
+        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, zero, st);
+        return launch_bwd<64, 4, 1, false, false, true>(a, vr, zero, st);
     }
     if (hd == 64) {
-        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, st);
-        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, st);
-        return launch_bwd<64, 4, 1>(a, vr, st);
+        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, zero, st);
+        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, zero, st);
+        return launch_bwd<64, 4, 1>(a, vr, zero, st);
     }
-    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, st);
-    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, st);
-    return launch_bwd<32, 4, 2>(a, vr, st);
+    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, zero, st);
+    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, zero, st);
+    return launch_bwd<32, 4, 2>(a, vr, zero, st);
 }
 
 extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
@@ -694,5 +793,5 @@ extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int6
                                 float* dE_k, float* dE_v, float* dW_pe, void* stream) {
     return mb_flash_ema_bwd_lists(Q, q_sb, q_sh, q_sl, q_sd, dO, x, x_sb, x_sl, E_k, E_v, W_pe, rhos, unique,
                                   C_bounds, O, LSE, B, H, L, hd, K, N, Np, nc, Br, V_total, flags, scores, dQ,
-                                  dE_k, dE_v, dW_pe, nullptr, stream);
+                                  dE_k, dE_v, dW_pe, nullptr, nullptr, 0, stream);
 }

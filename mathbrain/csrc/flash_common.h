@@ -28,6 +28,8 @@
 
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
+
 #include "common.h"
 
 namespace mb {
@@ -93,6 +95,9 @@ struct FlashArgs {
     // [B, ntb] counts; a workgroup then walks its block's list instead of all K slots
     const BatchMeta* list;
     const SlotCount* nlist;
+    const int32_t* order;  // the blocks b * ntb + t by the length of their lists, longest first
+    int ksplit;  // backward: slot parts per (b, block, head group)
+    float* dWpart;  // backward: NULL (dW_pe by atomics), or each workgroup's own dW_pe sums
 };
 
 // Arguments of the kernels whose E_k / E_v (and dE_k / dE_v) rows are token ids into
@@ -106,6 +111,45 @@ template <> struct FlashArgsOf<true> { using type = FlashArgsV; };
 
 __device__ inline int64_t e_rows_of(const FlashArgs& a) { return (int64_t)a.B * a.K; }
 __device__ inline int64_t e_rows_of(const FlashArgsV& a) { return a.e_rows; }
+
+// Compute units of the current device (cached per device).
+inline int device_cus() {
+    static int cus[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    if (cus[dev] <= 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+            (void)hipGetLastError();
+            n = 256;
+        }
+        cus[dev] = n;
+    }
+    return cus[dev];
+}
+
+// Slot parts for G workgroups of up to nbatch slot batches on a device that holds `conc` at
+// once.  Splitting each workgroup's batches into ks runs fills the compute units that a small
+// grid leaves idle, and lets a grid of about one round even out the blocks' different lists and
+// its last round; each part repeats the prologue and epilogue (10 to 30 us; a batch is 2 to 4).
+// Half a round or less is split to one full round, or to two where that leaves at least 32
+// batches to a part; more than half a round and less than two to about four rounds of such
+// parts; beyond that the rounds even out by themselves.  Measured, backward + forward kernels:
+// B3 T201 H6 N33 in fp32 mode 356 + 96 -> 81 + 49 us; B2 T128 H4 N16 83 + 32 -> 27 + 24 us;
+// B8 T512 H8 of documents (0.5 and 1 rounds) two parts 2.57 + 2.57 ms, four 2.35 + 1.37 ms.
+constexpr int kPartsMax = 32;
+constexpr int kPartBatches = 32;
+inline int slot_parts(int64_t G, int64_t conc, int nbatch) {
+    if (G <= 0 || conc <= 0 || G >= 2 * conc) return 1;
+    const int64_t longest = nbatch / kPartBatches;
+    const int64_t parts = 2 * G <= conc ? std::max(std::min<int64_t>(conc / G, nbatch / 2),
+                                                   std::min<int64_t>(2 * conc / G, longest))
+                                        : std::min<int64_t>((4 * conc + G - 1) / G, longest);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(parts, kPartsMax));
+}
 
 // Sets a kernel's dynamic LDS limit and launches it with its arguments.
 template <class Kern, class... Args>
@@ -198,21 +242,25 @@ __device__ inline float row_sum16(float v) {
     return v;
 }
 
-// Workgroup id -> (sequence b, 32-step block t, index r < inner within them), the blocks from
-// the last to the first: a block's slot list grows with the steps before it, and the longest
-// workgroups first leave the shortest for the end, when the rounds run out of step (at B56 T512
-// the first-to-last order cost 0.8 of the forward's 11.2 ms: an eighth workgroup on a CU whose
-// others took seven).  With B a multiple of 8 each XCD keeps its own sequences (the dispatcher
-// hands workgroups to the 8 XCDs round-robin), whose slot embeddings then share its L2.
+// Workgroup id -> (sequence b, 32-step block t, index r < inner within them): the blocks in the
+// order of the lists' lengths, longest first (flash_slots.hip), or without lists from the last
+// to the first, so that the shortest are left for the end, when the rounds run out of step
+// (first to last cost 0.8 of the forward's 11.2 ms at B56 T512: an eighth workgroup on a CU whose
+// others took seven).  Neighbours go to different XCDs (the dispatcher hands workgroups to the 8
+// XCDs round-robin): given sequences of its own, whose slot embeddings would share its L2, an XCD
+// with short lists waits for one with long ones (B8 T512 of documents: backward 5.05 -> 3.37 ms,
+// forward 2.69 -> 1.84), and sharing did not pay where they are equally long either (B56 T512
+// 20.6 -> 20.5 ms without).
 struct FlashBlock {
     int b, t, r;
 };
-__device__ inline FlashBlock flash_block(int bid, int B, int ntb, int inner) {
-    const int xcds = B % 8 ? 1 : 8;
-    const int per = B / xcds;
-    const int l = bid / xcds;
-    const int q = l / inner;
-    return FlashBlock{bid % xcds * per + q % per, ntb - 1 - q / per, l % inner};
+__device__ inline FlashBlock flash_block(const FlashArgs& a, int id, int ntb, int inner) {
+    const int q = id / inner;
+    if (a.list) {
+        const int i = a.order[q];
+        return FlashBlock{i / ntb, i % ntb, id % inner};
+    }
+    return FlashBlock{q % a.B, ntb - 1 - q / a.B, id % inner};
 }
 
 // LDS carve-up of the per-batch staging buffers: cdec (fp16), with BF the transposed bf16
@@ -266,29 +314,26 @@ __device__ inline int64_t e_row(const A& a, int b, const BatchMeta& m) {
 // Token id as BatchMeta holds it: ids past 2^31 - 1 clamp (e_row clamps to the table anyway).
 __device__ inline int32_t slot_row(int64_t u) { return (int32_t)min(u, (int64_t)INT32_MAX); }
 
-// Per-workgroup setup shared by both kernels: the match window tokens, the rho^j table
-// (j = 0..64), kinfo[0] = the valid slots of sequence b and kinfo[1] = the slots to walk (the
-// length of the block's list, or without lists one past the last valid slot).
+// The rho^j table (j = 0..64): thread tid takes rate tid % NPAD, so its double-precision log2 is
+// evaluated once (threads past a whole multiple of NPAD repeat entries).
 template <int NPAD>
-__device__ void flash_setup(const FlashArgs& a, int b, int t0, int cb, int64_t* win,
-                            float* powt, int* kinfo) {
+__device__ void flash_powers(const FlashArgs& a, float* powt) {
+    const int n = threadIdx.x % NPAD;
+    float hi = 0.f, lo = 0.f;
+    if (n < a.N) log2_split(a.rhos[n], hi, lo);
+    for (int j = threadIdx.x / NPAD; j <= 64; j += blockDim.x / NPAD)
+        powt[j * NPAD + n] = n < a.N ? pow_steps(hi, lo, j) : 0.0f;
+}
+
+// Per-block setup shared by both kernels: the match window tokens, kinfo[0] = the valid slots of sequence b and kinfo[1] = the slots to walk (the
+// length of the block's list, or without lists one past the last valid slot).
+__device__ inline void flash_setup(const FlashArgs& a, int b, int t0, int cb, int64_t* win, int* kinfo) {
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
     for (int p = tid; p < kMaxWin; p += nthr) {
         const int pos = cb + p;
         win[p] = (pos < a.L && pos < t0 + kTB) ? a.x[(int64_t)b * a.x_sb + (int64_t)pos * a.x_sl]
                                               : (int64_t)-1;
-    }
-    for (int i = tid; i < 65 * NPAD; i += nthr) {
-        const int j = i / NPAD;
-        const int n = i % NPAD;
-        float v = 0.0f;
-        if (n < a.N) {
-            float hi, lo;
-            log2_split(a.rhos[n], hi, lo);
-            v = pow_steps(hi, lo, j);
-        }
-        powt[i] = v;
     }
     if (tid == 0) {
         kinfo[0] = 0;   // valid slots K_b

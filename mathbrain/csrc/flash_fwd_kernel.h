@@ -72,7 +72,7 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
     const int ntb = (a.L + kTB - 1) / kTB;
     // one workgroup per (b, 32-step block, slot part, head group); a group holds hpg heads
     // (hpg divides H), one wave each, and waves past hpg only help stage and synchronise
-    const FlashBlock blk = flash_block(blockIdx.x, a.B, ntb, sp.ksplit * a.head_groups);
+    const FlashBlock blk = flash_block(a, blockIdx.x, ntb, sp.ksplit * a.head_groups);
     const int hg = blk.r % a.head_groups;
     const int part = blk.r / a.head_groups;
     const int t0 = blk.t * kTB;
@@ -119,7 +119,8 @@ flash_ema_fwd_kernel(typename FlashArgsK<VR, GQ>::type a, FwdSplit sp) {
         __syncthreads();
     }
 
-    flash_setup<NPAD>(a, b, t0, cb, win, powt, kinfo);
+    flash_powers<NPAD>(a, powt);
+    flash_setup(a, b, t0, cb, win, kinfo);
     const int kvalid = kinfo[0];
     const int kend = kinfo[1];
     // this part's batches [bi0, bi1)
@@ -429,33 +430,12 @@ flash_fwd_merge_kernel(const float* __restrict__ part, int ks, int64_t rows, flo
     if (c == 0) LSE[r] = any ? (M + __log2f(l)) * kLn2 : -INFINITY;
 }
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
-    static int cus[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    if (cus[dev] <= 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-            (void)hipGetLastError();
-            n = 256;
-        }
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
-
-// Slot parts per workgroup of the forward.  The workgroups of one launch run in rounds of
-// `conc` (all that the device holds at once) and take about equally long, so G of them
-// take ceil(G / conc) rounds: 896 at configuration 2 take 4 rounds of 256 where 3.5 would
-// do.  Splitting each workgroup's slot batches into ks parts gives G ks workgroups of
-// 1 / ks the length; a split must save at least 3 % (each part repeats the prologue and
-// its state goes through the merge) and keep at least four batches per part.
+// Slot parts of the forward: slot_parts for a grid below two rounds of `conc` workgroups.
+// Beyond that the workgroups of equally long lists end their rounds together, and a split
+// must save at least 3 % of the rounds: 896 at B56 T512 take 4 rounds of 256 where 3.5 would
+// do (two parts: 10.22 -> 9.12 ms with single products), and keep four batches per part.
 static int fwd_parts(int64_t G, int64_t conc, int nbatch) {
-    if (G <= 0 || conc <= 0) return 1;
+    if (G < 2 * conc) return slot_parts(G, conc, nbatch);
     int best = 1;
     double best_cost = (double)((G + conc - 1) / conc);
     for (int ks = 2; ks <= 4; ++ks) {

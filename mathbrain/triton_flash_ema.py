@@ -396,12 +396,15 @@ def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V
     with torch.cuda.device(dev):
         if lists is None:
             lists = _slot_lists(xl, uniq, Cb, N, Br)
+        nws = int(_lib.lib().mb_flash_ema_bwd_workspace(hd, N))
+        ws = torch.empty(nws, dtype=torch.uint8, device=dev)
         _lib.call("mb_flash_ema_bwd_lists", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(dOf), _lib.ptr(xl),
                   xl.stride(0), xl.stride(1), _lib.ptr(Ek), _lib.ptr(Ev), _lib.ptr(W),
                   _lib.ptr(rh), _lib.ptr(uniq), _lib.ptr(Cb), _lib.ptr(Of), _lib.ptr(Lf), B, H, L,
                   hd, K, N, Cb.shape[3], Cb.shape[1], int(Br), int(V_total),
                   _flash_flags(use_silu, absent_mass, table, prec), _lib.ptr(scores), _lib.ptr(dQ),
-                  _lib.ptr(dEk), _lib.ptr(dEv), _lib.ptr(dW), _lib.ptr(lists), _lib.stream(dev))
+                  _lib.ptr(dEk), _lib.ptr(dEv), _lib.ptr(dW), _lib.ptr(lists), _lib.ptr(ws), nws,
+                  _lib.stream(dev))
     return dQ, dEk, dEv, dW
 
 

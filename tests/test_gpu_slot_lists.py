@@ -62,7 +62,7 @@ def call(c, dev, lists, absent_mass, use_silu, prec):
     outs = []
     for scores in (S2, None):
         _lib.call("mb_flash_ema_bwd_lists", p(Q), *Q.stride(), p(dO), p(x), x.stride(0), x.stride(1), p(Ek), p(Ev),
-                  p(W), p(rh), p(u), p(Cb), p(O), p(LSE), *common, p(scores), *(p(t) for t in g), p(lists), st)
+                  p(W), p(rh), p(u), p(Cb), p(O), p(LSE), *common, p(scores), *(p(t) for t in g), p(lists), None, 0, st)
         outs += [t.cpu() for t in g]
     return [O.cpu(), LSE.cpu()] + outs
 
@@ -83,11 +83,16 @@ def test_lists_and_the_attention_over_them(L, N, Br, warmup, pad_slots, absent_m
     buf = lists_of(c, dev)
     nblk = -(-L // 32)
     entries = buf[:B * nblk * K * 16].view(torch.int32).view(B, nblk, K, 4).cpu()
-    counts = buf[B * nblk * K * 16:].view(torch.int32).view(B, nblk, 2).cpu()
+    counts = buf[B * nblk * K * 16:-B * nblk * 4].view(torch.int32).view(B, nblk, 2).cpu()
+    order = buf[-B * nblk * 4:].view(torch.int32).cpu()
     for (b, blk), ks in expected(c).items():
         assert counts[b, blk].tolist() == [len(ks), int((c["unique"][b] >= 0).sum())]
         assert entries[b, blk, :len(ks), 3].tolist() == ks
         assert entries[b, blk, :len(ks), 2].tolist() == c["unique"][b, ks].tolist()
+    # every block once, the longest lists first (to within a 1023rd of K)
+    assert sorted(order.tolist()) == list(range(B * nblk))
+    ordered = counts.view(-1, 2)[order.long(), 0]
+    assert bool((ordered[1:] - ordered[:-1] <= K / 1023 + 1).all())
     for use_silu, prec in ((True, "bf16"), (False, "fp32" if N <= 64 else "fp16")):
         got = call(c, dev, buf, absent_mass, use_silu, prec)
         want = call(c, dev, None, absent_mass, use_silu, prec)
