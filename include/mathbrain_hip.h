@@ -399,6 +399,20 @@ int mb_gating_bwd(const float *dy, const float *x_q, int64_t xq_row_stride, cons
                   void *stream);
 
 /*
+ * Weight gradient of the folded projection: dW[n,d] = sum_r (C_seq[r,n] + 1) dpre[r,d], what the
+ * autograd of pe_proj and of its row sum gives W_pe = pe_proj.weight transposed
+ * (mathbrain/triton_fused_gating.py:179-186).  fp32 products and sums.
+ *
+ *   dpre      [rows, D] fp32 contiguous (mb_gating_bwd's dp_pre)
+ *   C_seq     [rows, N] fp32, row stride c_row_stride
+ *   workspace mb_gating_dw_workspace(rows, N, D) bytes of device memory (0: may be NULL)
+ *   dW        [N, D] fp32 contiguous output
+ */
+int64_t mb_gating_dw_workspace(int64_t rows, int N, int D);
+int mb_gating_dw(const float *dpre, const float *C_seq, int64_t c_row_stride, int64_t rows, int N,
+                 int D, void *workspace, int64_t workspace_bytes, float *dW, void *stream);
+
+/*
  * Data pipeline on the device (the producers of the hot path's inputs).
  *
  * Per-position EMA states of a whole corpus.  Replaces the preprocessing scan of

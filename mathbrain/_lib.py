@@ -54,6 +54,8 @@ SIGNATURES = {
                        _p, _p, _p], _i),
     "mb_gating_bwd": ([_p, _p, _i64, _p, _i64, _p, _p, _i64, _p, _i, _p, _p, _p, _i64, _i, _i, _p,
                        _p, _p, _p, _p, _p], _i),
+    "mb_gating_dw_workspace": ([_i64, _i, _i], _i64),
+    "mb_gating_dw": ([_p, _p, _i64, _i64, _i, _i, _p, _i64, _p, _p], _i),
     "mb_corpus_states_workspace": ([_i64, _i], _i64),
     "mb_corpus_states": ([_p, _p, _i64, _p, _i, _p, _p, _i64, _p], _i),
     "mb_corpus_states_noalloc": ([_p, _p, _i64, _p, _i, _p, _p], _i),

@@ -686,7 +686,7 @@ class GatedQueryFlashEMAFunction(torch.autograd.Function):
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, dO):
-        from .triton_fused_gating import gating_bwd, gating_fwd
+        from .triton_fused_gating import gating_bwd, gating_dw, gating_fwd
         (x_q, C_seq, W_pe, ln_w, ln_b, W_q, x, E_k, E_v, rhos, unique_tensor, C_bounds, O,
          LSE) = ctx.saved_tensors
         V_total, use_silu, Br, absent_mass, prec, eps, H = ctx.cfg
@@ -702,11 +702,9 @@ class GatedQueryFlashEMAFunction(torch.autograd.Function):
         dQr = dQ.transpose(1, 2).reshape(B * L, D)  # row (b, t), column h hd + d
         dW_q = dQr.t() @ xr
         dx_ln = dQr @ W_q
-        dxq, dpre, dbias, dlnw, dlnb = gating_bwd(dx_ln.view(B, L, D), x_q, None, None, C_seq, Wpe, ln_w,
-                                                  mu, rstd, use_silu)
-        # the gate's weight gradient: sum_r (C_seq[r] + 1)^T dpre[r] (the bias term's column sum
-        # came reduced from the kernel), plus the attention's
-        dW = torch.addmm(dbias.unsqueeze(0).expand(N, D), C_seq.reshape(-1, N).t(), dpre) + dWa
+        dxq, dpre, _, dlnw, dlnb = gating_bwd(dx_ln.view(B, L, D), x_q, None, None, C_seq, Wpe, ln_w, mu,
+                                              rstd, use_silu)
+        dW = gating_dw(C_seq, dpre) + dWa  # the gate's weight gradient and the attention's
         if W_pe.shape[0] > N:  # W_pe passed with padded rows: their gradient is 0
             dW = torch.cat([dW, dW.new_zeros(W_pe.shape[0] - N, D)])
         dC = (dpre @ Wpe.t()).reshape(C_seq.shape) if ctx.needs_input_grad[1] else None

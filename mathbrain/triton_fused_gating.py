@@ -130,6 +130,28 @@ def gating_bwd(dy: torch.Tensor, x_q: torch.Tensor, p_pre: Optional[torch.Tensor
     return dxq, dpre, dbias, dlnw, dlnb
 
 
+def _gate_dw_fake(C_seq, dpre):
+    return dpre.new_empty((C_seq.shape[-1], dpre.shape[1]))
+
+
+@_lib.traced_op("gating_dw", _gate_dw_fake)
+def gating_dw(C_seq: torch.Tensor, dpre: torch.Tensor) -> torch.Tensor:
+    """dW_pe [N, D] = (C_seq + 1)^T dpre, the folded projection's weight gradient, from dpre
+    [rows, D] (mb_gating_dw: one launch, and one that adds the row parts' sums)."""
+    dev = _lib.require_gpu(C_seq, dpre, what="query gating")
+    N = C_seq.shape[-1]
+    cs, css = _rows(C_seq.to(torch.float32), N)
+    g = dpre.to(torch.float32).contiguous()
+    rows, D = g.shape
+    dW = torch.empty(N, D, dtype=torch.float32, device=dev)
+    nws = int(_lib.lib().mb_gating_dw_workspace(rows, N, D))
+    ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
+    with torch.cuda.device(dev):
+        _lib.call("mb_gating_dw", _lib.ptr(g), _lib.ptr(cs), css, rows, N, D, _lib.ptr(ws), nws, _lib.ptr(dW),
+                  _lib.stream(dev))
+    return dW
+
+
 class FusedGatingFunction(torch.autograd.Function):
     """apply(x_q, p_pre, bias, ln_w, ln_b, use_silu=True) -> x_ln [B, L, D]
     (triton_fused_gating.py:122-177): LayerNorm_{1e-5}(x_q * SiLU(p_pre + bias)).
@@ -173,14 +195,10 @@ class GatedQueryFunction(torch.autograd.Function):
     @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx, dy):
         x_q, C_seq, W_pe, ln_w, mu, rstd, pre = ctx.saved_tensors
-        dxq, dpre, dbias, dlnw, dlnb = gating_bwd(dy, x_q, pre, None, None, None, ln_w, mu, rstd,
-                                                  ctx.use_silu)
-        N, D = W_pe.shape
+        dxq, dpre, _, dlnw, dlnb = gating_bwd(dy, x_q, pre, None, None, None, ln_w, mu, rstd, ctx.use_silu)
         dW = None
         if ctx.needs_input_grad[2]:
-            # dW[n, d] = sum_r (C[r, n] + 1) dpre[r, d]: a plain GEMM (K = rows) plus the
-            # bias term's column sum, which the kernel already reduced.
-            dW = torch.addmm(dbias.unsqueeze(0).expand(N, D), C_seq.reshape(-1, N).t(), dpre)
+            dW = gating_dw(C_seq, dpre)
         dC = None
         if ctx.needs_input_grad[1]:
             dC = (dpre @ W_pe.t()).reshape(C_seq.shape)

@@ -125,3 +125,21 @@ def test_empty_rows():
                                  torch.zeros(8, 64, device="cuda"), torch.ones(64, device="cuda"),
                                  torch.zeros(64, device="cuda"))
     assert y.shape == (0, 5, 64)
+
+
+@pytest.mark.parametrize("rows,D,N", [(1, 32, 1), (127, 33, 16), (257, 200, 7), (1000, 1000, 70), (4099, 512, 64),
+                                      (2050, 129, 128), (28673, 96, 65)])
+def test_projection_weight_gradient(rows, D, N):
+    """mb_gating_dw in one run of rows and in several, at the edges of its tiles (64 rates, 128
+    columns, steps of 4 and 16 rows), C_seq as rows of a wider matrix.  Bound: fp32 products and
+    sums of n terms are within n 2^-24 of the exact result relative to sum |C + 1| |dpre|
+    (elementwise); the longest chain here is the rows of a run plus the runs, under 2^11."""
+    from mathbrain.triton_fused_gating import gating_dw
+    g = torch.Generator().manual_seed(rows + D + N)
+    wide = torch.rand(rows, N + 3, generator=g) * 30
+    dpre = torch.randn(rows, D, generator=g)
+    C = wide[:, 2:2 + N]
+    got = gating_dw(wide.cuda()[:, 2:2 + N], dpre.cuda()).double().cpu()
+    want = (C.double() + 1).t() @ dpre.double()
+    size = (C.double() + 1).t() @ dpre.double().abs()
+    assert bool(((got - want).abs() <= 2.0 ** -13 * size).all())
