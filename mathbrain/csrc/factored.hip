@@ -13,9 +13,9 @@
 //
 // The kernels: fac_outer (scaled outer-product accumulation, builds S_n and the backward's
 // M_n = sum_t rho_n^(t+1) q_t ⊗ dO_t), fac_apply (contracts such a state with rows: the
-// c_base part of o, of dQ and of the slot gradients), and the three token-pair kernels
-// (forward; backward by rows for dQ, by columns for the token embedding gradients, by
-// diagonals for dG[d], from which dW_pe = P dG with P[n,d] = rho_n^d).
+// c_base part of o, of dQ and of the slot gradients), and the token-pair kernels: fac_tok_pair
+// (o, and the token gradients of e_v), fac_tok_gate (dQ, and the token gradients of e_k) and
+// fac_tok_dist (dG[d], from which dW_pe = P dG with P[n,d] = rho_n^d).
 #include "flash_common.h"
 
 namespace mb {
@@ -375,309 +375,331 @@ __device__ inline bool tok_ok(int64_t v, int64_t V) { return v >= 0 && v < V; }
 
 // ---- token pairs ---------------------------------------------------------------------------
 //
-// The four kernels share one shape.  A block of 4 waves covers 64 steps of one (b, h) on its
-// lanes (the "lane steps") and walks the 64-step blocks of the other index (the "walked
-// steps"); the 4 waves take every fourth walked step and their partial sums are added in LDS
-// at the end.  Each tile stages in LDS the rows of its walked block (q, dO, e_k or e_v: one
-// row for the whole wave, read by every lane at the same address) and the 127
-// distance-dependent G rows it needs (a different row per lane).  Each lane holds whole
-// hd-rows in registers, so no cross-lane sums are needed per pair.
+// A block of 4 waves covers 64 steps (the "rows") of one (b, h) and walks the 64-step blocks of
+// the other index (the "walked" steps); wave w has rows 16 w .. 16 w + 15.  What a 64 x 64 tile
+// of pairs needs is one of two forms:
+//
+//   sums over the dimensions of a product of three rows, A[t,s] = sum_i q_t[i] e_k[x_s][i]
+//   G[t-s][i]: a thread takes 4 x 4 pairs and walks the dimensions, whose rows are staged with
+//   the dimension as the slow index; the 4 x 4 pairs have 7 distances, 8 consecutive floats;
+//
+//   sums over the walked steps of dA[r,w] y_w ⊙ G[d]: a thread takes 4 rows x 4 dimensions (2 x 4
+//   at head_dim 32) and walks the steps; its rows' distances move by one per step, so a step
+//   reads one new row of G.
+//
+// The products without G (A e_v, dO e_v^T, A^T dO) go to the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32: A[row = lane % 16][k = lane / 16], B[k = lane / 16][col = lane % 16],
+// D[row = 4 (lane / 16) + i][col = lane % 16]).  Bound: VALU issue, two operations per pair and
+// dimension (A in the forward and for dE_v, dQ, dE_k and dG: 10 in all), and next to it the LDS
+// reads, 3 or 4 of 16 bytes per 32 operations.  Lanes as steps with whole rows in registers
+// instead read G from LDS for every pair and dimension, and the other rows once per wave.
+// B56 T512 H8 head_dim 64, forward + backward: 9.4 -> 4.25 ms (o 0.78, dE_v 0.74, dQ 0.84,
+// dE_k 0.82, dG 1.08); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.61 ms.
 
-constexpr int kTW = 4;  // waves per block
+constexpr int kTokB = 64;  // steps per block
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int HD>
-struct TokLds {
-    static constexpr int RS = HD + 4;  // padded row stride (floats) of the staged rows
-    static constexpr int GROWS = 127;
+// Rows of one head: of a [L, D] slice (ids NULL), or E[x[r]] of a table; rows outside [0, L) and
+// ids outside [0, V) read as zeros.
+struct TokRows {
+    const float* p;
+    const int64_t* ids;
+    int64_t V, D;
+    int L;
+    __device__ inline const float* row(int r) const {
+        if (r < 0 || r >= L) return nullptr;
+        if (!ids) return p + r * D;
+        const int64_t v = ids[r];
+        return tok_ok(v, V) ? p + v * D : nullptr;
+    }
 };
 
-// Stages rows [lo, lo + n) of a [rows_total, D] table (head slice h) into dst with stride RS;
-// rows outside [0, rows_total) are zero.
-template <int HD>
-__device__ inline void stage_rows(float* dst, const float* src, int64_t D, int h, int lo, int n,
-                                  int rows_total) {
-    constexpr int RS = TokLds<HD>::RS;
+__device__ inline f32x4 load4(const float* p, int c) {
+    return p ? f32x4(*reinterpret_cast<const f32x4u*>(p + c)) : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// dst[k][r] = rows lo + r, dimensions k0 + k, for ROWS x KC; RS floats per dimension.  Four lanes
+// on 64 bytes of a row and 16 rows per wave: the transposed writes use every bank twice.
+template <int ROWS, int KC, int RS>
+__device__ inline void stage_by_dim(float* dst, const TokRows& src, int lo, int k0) {
+    const int cl = threadIdx.x & 3, rl = (threadIdx.x >> 2) & 15, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int rest = 0; rest < (ROWS / 16) * (KC / 16); rest += 4) {
+        const int r = ((rest + wave) % (ROWS / 16)) * 16 + rl;
+        const int c = ((rest + wave) / (ROWS / 16)) * 16 + 4 * cl;
+        const f32x4 v = load4(src.row(lo + r), k0 + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[(c + e) * RS + r] = v[e];
+    }
+}
+
+// dst[r][i] = row lo + r, RS floats per row.
+template <int ROWS, int HD, int RS>
+__device__ inline void stage_by_row(float* dst, const TokRows& src, int lo) {
     constexpr int C4 = HD / 4;
-    for (int e = threadIdx.x; e < n * C4; e += 64 * kTW) {
-        const int r = e / C4, c = e % C4;
-        const int row = lo + r;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (row >= 0 && row < rows_total)
-            v = *reinterpret_cast<const float4*>(src + (int64_t)row * D + h * HD + 4 * c);
-        *reinterpret_cast<float4*>(dst + r * RS + 4 * c) = v;
-    }
-}
-
-// Same for token-indexed rows: row r is E[x[b, lo + r]] (zero outside [0, L) or for ids
-// outside [0, V)).
-template <int HD>
-__device__ inline void stage_tok_rows(float* dst, const float* E, const int64_t* xb, int64_t V,
-                                      int64_t D, int h, int lo, int n, int L) {
-    constexpr int RS = TokLds<HD>::RS;
-    constexpr int C4 = HD / 4;
-    for (int e = threadIdx.x; e < n * C4; e += 64 * kTW) {
-        const int r = e / C4, c = e % C4;
-        const int s = lo + r;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (s >= 0 && s < L) {
-            const int64_t xs = xb[s];
-            if (tok_ok(xs, V)) v = *reinterpret_cast<const float4*>(E + xs * D + h * HD + 4 * c);
-        }
-        *reinterpret_cast<float4*>(dst + r * RS + 4 * c) = v;
-    }
-}
-
-// Adds the kTW waves' per-lane rows acc[HD] in LDS (red holds (kTW-1)*64*HD floats) and
-// leaves the sum in wave 0.
-template <int HD>
-__device__ inline void reduce_waves(float (&acc)[HD], float* red) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    __syncthreads();
-    if (w > 0) {
 #pragma unroll
-        for (int k = 0; k < HD; ++k) red[((w - 1) * HD + k) * 64 + lane] = acc[k];
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-        for (int k = 0; k < HD; ++k) {
-#pragma unroll
-            for (int v = 0; v < kTW - 1; ++v) acc[k] += red[(v * HD + k) * 64 + lane];
-        }
+    for (int e0 = 0; e0 < ROWS * C4; e0 += 256) {
+        const int e = e0 + threadIdx.x, r = e / C4, c = 4 * (e % C4);
+        *reinterpret_cast<f32x4*>(dst + r * RS + c) = load4(src.row(lo + r), c);
     }
 }
 
-// LDS of a token-pair block: the tile's 127 distance rows plus the walked block's two row
-// sets (64 rows each), or the wave partials at the end.
-template <int HD>
-constexpr int tok_lds_floats() {
-    constexpr int a = (TokLds<HD>::GROWS + 2 * 64) * TokLds<HD>::RS;
-    constexpr int r = (kTW - 1) * 64 * HD;
-    return a > r ? a : r;
-}
-
-// Forward token part (lanes = steps t, walked = steps s < t):
-//   O[b,t,h,:] = sum_{s<t} (sum_i q_t[i] e_k[x_s][i] G[t-s][i]) e_v[x_s].
-template <int HD>
-__global__ void __launch_bounds__(64 * kTW)
-fac_tok_fwd_kernel(const float* __restrict__ Q, const int64_t* __restrict__ x, int64_t V,
-                   const float* __restrict__ Ek, const float* __restrict__ Ev,
-                   const float* __restrict__ G, int L, int H, float* __restrict__ O) {
-    constexpr int RS = TokLds<HD>::RS;
-    __shared__ __align__(16) float lds[tok_lds_floats<HD>()];
+// out[r] = sum_w A(r, w) Z[w], A(r, w) = sum_i X[r][i] Y[w][i] G[d][i].  FWD: rows are steps t
+// and the walked ones s < t (O); otherwise rows are steps s and the walked ones t > s (dE_v).
+template <int HD, bool FWD>
+__global__ void __launch_bounds__(256, 2)
+fac_tok_pair_kernel(const float* __restrict__ Q, const float* __restrict__ dO, const int64_t* __restrict__ x,
+                    int64_t V, const float* __restrict__ Ek, const float* __restrict__ Ev,
+                    const float* __restrict__ G, int L, int H, float* __restrict__ out) {
+    constexpr int KC = 32;        // dimensions per staged piece of Y and G
+    constexpr int RS = kTokB + 4;   // floats per dimension of 64 rows, and of an A row
+    constexpr int GS = 2 * kTokB + 4;
+    constexpr int ZS = HD + 16;   // the four k groups of an operand read on different banks
+    __shared__ __align__(16) float Xs[HD * RS], Ys[KC * RS], Gs[KC * GS], As[kTokB * RS], Zs[kTokB * ZS];
     const int64_t D = (int64_t)H * HD;
-    const int b = blockIdx.z, h = blockIdx.y, tb = blockIdx.x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int t = tb * 64 + lane;
-    const bool tv = t < L;
+    const int b = blockIdx.z, h = blockIdx.y, nb = gridDim.x;
+    const int rb = FWD ? nb - 1 - (int)blockIdx.x : (int)blockIdx.x;  // most walked blocks first
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int ty = tid >> 4, tx = tid & 15;
+    const int c16 = lane & 15, g = lane >> 4;
     const int64_t* xb = x + (int64_t)b * L;
-    float q[HD], o[HD];
+    const int64_t slice = (int64_t)b * L * D + h * HD;
+    const TokRows q{Q + slice, nullptr, 0, D, L}, ek{Ek + h * HD, xb, V, D, L};
+    const TokRows z = FWD ? TokRows{Ev + h * HD, xb, V, D, L} : TokRows{dO + slice, nullptr, 0, D, L};
+    const TokRows gt{G + h * HD, nullptr, 0, D, L + 1};
+    const TokRows xr = FWD ? q : ek, yr = FWD ? ek : q;
+    f32x4 acc[HD / 16];
 #pragma unroll
-    for (int k = 0; k < HD; ++k) {
-        q[k] = tv ? Q[((int64_t)b * L + t) * D + h * HD + k] : 0.0f;
-        o[k] = 0.0f;
-    }
-    float* sk = lds + TokLds<HD>::GROWS * RS;  // e_k rows of the walked block
-    float* sv = sk + 64 * RS;                   // e_v rows
-    for (int sb = 0; sb <= tb; ++sb) {
-        const int dlo = (tb - sb) * 64 - 63;
-        __syncthreads();
-        stage_rows<HD>(lds, G, D, h, dlo, TokLds<HD>::GROWS, L + 1);
-        stage_tok_rows<HD>(sk, Ek, xb, V, D, h, sb * 64, 64, L);
-        stage_tok_rows<HD>(sv, Ev, xb, V, D, h, sb * 64, 64, L);
-        __syncthreads();
-        const int s_hi = min(sb * 64 + 64, L);
-        for (int s = sb * 64 + w; s < s_hi; s += kTW) {
-            const float* ek = sk + (s - sb * 64) * RS;
-            const float* ev = sv + (s - sb * 64) * RS;
-            const int di = t - s - dlo;
-            const bool pair = tv && t > s;
-            const float* g = lds + (pair ? di : 0) * RS;
-            float a = 0.0f;
+    for (int j = 0; j < HD / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    stage_by_dim<kTokB, HD, RS>(Xs, xr, rb * kTokB, 0);
+    const float* gbase = Gs + (FWD ? 4 * (ty - tx) : 4 * (tx - ty)) + 60;
+    const int w_lo = FWD ? 0 : rb, w_hi = FWD ? rb : nb - 1;
+    for (int wb = w_lo; wb <= w_hi; ++wb) {
+        const int dlo = (FWD ? rb - wb : wb - rb) * kTokB - (kTokB - 1);
+        float a[4][4];
 #pragma unroll
-            for (int k = 0; k < HD; ++k) a = __builtin_fmaf(q[k] * ek[k], g[k], a);
-            a = pair ? a : 0.0f;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int k = 0; k < HD; ++k) o[k] = __builtin_fmaf(a, ev[k], o[k]);
-        }
-    }
-    reduce_waves<HD>(o, lds);
-    if (w == 0 && tv) {
+            for (int j = 0; j < 4; ++j) a[i][j] = 0.f;
 #pragma unroll
-        for (int k = 0; k < HD; ++k) O[((int64_t)b * L + t) * D + h * HD + k] = o[k];
-    }
-}
-
-// Backward by rows (lanes = t, walked = s < t): dQ[b,t,h,:] = sum_{s<t} (dO_t . e_v[x_s])
-// e_k[x_s] ⊙ G[t-s].
-template <int HD>
-__global__ void __launch_bounds__(64 * kTW)
-fac_tok_bwd_row_kernel(const float* __restrict__ dO, const int64_t* __restrict__ x, int64_t V,
-                       const float* __restrict__ Ek, const float* __restrict__ Ev,
-                       const float* __restrict__ G, int L, int H, float* __restrict__ dQ) {
-    constexpr int RS = TokLds<HD>::RS;
-    __shared__ __align__(16) float lds[tok_lds_floats<HD>()];
-    const int64_t D = (int64_t)H * HD;
-    const int b = blockIdx.z, h = blockIdx.y, tb = blockIdx.x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int t = tb * 64 + lane;
-    const bool tv = t < L;
-    const int64_t* xb = x + (int64_t)b * L;
-    float go[HD], dq[HD];
+        for (int kc = 0; kc < HD; kc += KC) {
+            __syncthreads();
+            stage_by_dim<kTokB, KC, RS>(Ys, yr, wb * kTokB, kc);
+            stage_by_dim<2 * kTokB, KC, GS>(Gs, gt, dlo, kc);
+            if (kc == 0) stage_by_row<kTokB, HD, ZS>(Zs, z, wb * kTokB);
+            __syncthreads();
+#pragma unroll 4
+            for (int k = 0; k < KC; ++k) {
+                const f32x4 xv = *reinterpret_cast<const f32x4*>(Xs + (kc + k) * RS + 4 * ty);
+                const f32x4 yv = *reinterpret_cast<const f32x4*>(Ys + k * RS + 4 * tx);
+                const f32x4 g0 = *reinterpret_cast<const f32x4*>(gbase + k * GS);
+                const f32x4 g1 = *reinterpret_cast<const f32x4*>(gbase + k * GS + 4);
+                const float gg[8] = {g0[0], g0[1], g0[2], g0[3], g1[0], g1[1], g1[2], g1[3]};
 #pragma unroll
-    for (int k = 0; k < HD; ++k) {
-        go[k] = tv ? dO[((int64_t)b * L + t) * D + h * HD + k] : 0.0f;
-        dq[k] = 0.0f;
-    }
-    float* sk = lds + TokLds<HD>::GROWS * RS;
-    float* sv = sk + 64 * RS;
-    for (int sb = 0; sb <= tb; ++sb) {
-        const int dlo = (tb - sb) * 64 - 63;
-        __syncthreads();
-        stage_rows<HD>(lds, G, D, h, dlo, TokLds<HD>::GROWS, L + 1);
-        stage_tok_rows<HD>(sk, Ek, xb, V, D, h, sb * 64, 64, L);
-        stage_tok_rows<HD>(sv, Ev, xb, V, D, h, sb * 64, 64, L);
-        __syncthreads();
-        const int s_hi = min(sb * 64 + 64, L);
-        for (int s = sb * 64 + w; s < s_hi; s += kTW) {
-            const float* ek = sk + (s - sb * 64) * RS;
-            const float* ev = sv + (s - sb * 64) * RS;
-            const int di = t - s - dlo;
-            const bool pair = tv && t > s;
-            const float* g = lds + (pair ? di : 0) * RS;
-            float da = 0.0f;
+                for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int k = 0; k < HD; ++k) da = __builtin_fmaf(go[k], ev[k], da);
-            da = pair ? da : 0.0f;
-#pragma unroll
-            for (int k = 0; k < HD; ++k) dq[k] = __builtin_fmaf(da * ek[k], g[k], dq[k]);
-        }
-    }
-    reduce_waves<HD>(dq, lds);
-    if (w == 0 && tv) {
-#pragma unroll
-        for (int k = 0; k < HD; ++k) dQ[((int64_t)b * L + t) * D + h * HD + k] = dq[k];
-    }
-}
-
-// Backward by columns (lanes = s, walked = t > s).  KEY = true: dEk_tok[b,s,h,:] =
-// sum_{t>s} (dO_t . e_v[x_s]) q_t ⊙ G[t-s]; KEY = false: dEv_tok[b,s,h,:] =
-// sum_{t>s} (sum_i q_t[i] e_k[x_s][i] G[t-s][i]) dO_t.
-template <int HD, bool KEY>
-__global__ void __launch_bounds__(64 * kTW)
-fac_tok_bwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ dO,
-                       const int64_t* __restrict__ x, int64_t V, const float* __restrict__ Ek,
-                       const float* __restrict__ Ev, const float* __restrict__ G, int L, int H,
-                       float* __restrict__ out) {
-    constexpr int RS = TokLds<HD>::RS;
-    __shared__ __align__(16) float lds[tok_lds_floats<HD>()];
-    const int64_t D = (int64_t)H * HD;
-    const int b = blockIdx.z, h = blockIdx.y, sb = blockIdx.x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int s = sb * 64 + lane;
-    bool sv = s < L;
-    const int64_t xs = sv ? x[(int64_t)b * L + s] : 0;
-    sv = sv && tok_ok(xs, V);
-    const float* E = KEY ? Ev : Ek;  // the row this lane keeps: e_v for dA, e_k for A
-    float e[HD], acc[HD];
-#pragma unroll
-    for (int k = 0; k < HD; ++k) {
-        e[k] = sv ? E[xs * D + h * HD + k] : 0.0f;
-        acc[k] = 0.0f;
-    }
-    const int nb = (L + 63) / 64;
-    float* sq = lds + TokLds<HD>::GROWS * RS;  // q rows of the walked block
-    float* so = sq + 64 * RS;                   // dO rows
-    for (int tb = sb; tb < nb; ++tb) {
-        const int dlo = (tb - sb) * 64 - 63;
-        __syncthreads();
-        stage_rows<HD>(lds, G, D, h, dlo, TokLds<HD>::GROWS, L + 1);
-        stage_rows<HD>(sq, Q + (int64_t)b * L * D, D, h, tb * 64, 64, L);
-        stage_rows<HD>(so, dO + (int64_t)b * L * D, D, h, tb * 64, 64, L);
-        __syncthreads();
-        const int t_hi = min(tb * 64 + 64, L);
-        for (int t = tb * 64 + w; t < t_hi; t += kTW) {
-            const float* q = sq + (t - tb * 64) * RS;
-            const float* go = so + (t - tb * 64) * RS;
-            const int di = t - s - dlo;
-            const bool pair = sv && t > s;
-            const float* g = lds + (pair ? di : 0) * RS;
-            if (KEY) {
-                float da = 0.0f;
-#pragma unroll
-                for (int k = 0; k < HD; ++k) da = __builtin_fmaf(go[k], e[k], da);
-                da = pair ? da : 0.0f;
-#pragma unroll
-                for (int k = 0; k < HD; ++k) acc[k] = __builtin_fmaf(da * q[k], g[k], acc[k]);
-            } else {
-                float a = 0.0f;
-#pragma unroll
-                for (int k = 0; k < HD; ++k) a = __builtin_fmaf(q[k] * e[k], g[k], a);
-                a = pair ? a : 0.0f;
-#pragma unroll
-                for (int k = 0; k < HD; ++k) acc[k] = __builtin_fmaf(a, go[k], acc[k]);
+                    for (int j = 0; j < 4; ++j)
+                        a[i][j] = __builtin_fmaf(xv[i] * yv[j], gg[(FWD ? i - j : j - i) + 3], a[i][j]);
             }
         }
-    }
-    reduce_waves<HD>(acc, lds);
-    if (w == 0 && s < L) {
+        if (wb == rb || wb == nb - 1) {
 #pragma unroll
-        for (int k = 0; k < HD; ++k) out[((int64_t)b * L + s) * D + h * HD + k] = acc[k];
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int r = rb * kTokB + 4 * ty + i, w = wb * kTokB + 4 * tx + j;
+                    a[i][j] = (FWD ? r > w : w > r) && w < L ? a[i][j] : 0.f;
+                }
+        }
+        // the wave's 16 rows of A, written and read by the same wave
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<f32x4*>(As + (4 * ty + i) * RS + 4 * tx) = f32x4{a[i][0], a[i][1], a[i][2], a[i][3]};
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 4
+        for (int k = 0; k < kTokB / 4; ++k) {
+            const float av = As[(16 * wave + c16) * RS + 4 * k + g];
+#pragma unroll
+            for (int j = 0; j < HD / 16; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, Zs[(4 * k + g) * ZS + 16 * j + c16], acc[j], 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = rb * kTokB + 16 * wave + 4 * g + i;
+        if (r >= L) continue;
+        const bool ok = FWD || ek.row(r);
+#pragma unroll
+        for (int j = 0; j < HD / 16; ++j) out[slice + (int64_t)r * D + 16 * j + c16] = ok ? acc[j][i] : 0.f;
     }
 }
 
-// Backward by diagonals (lanes = distances d, walked = t): dGb[b,d,h,:] =
-// sum_t (dO_t . e_v[x_{t-d}]) q_t ⊙ e_k[x_{t-d}] for d in [1, L); row 0 is zero.  The e_k /
-// e_v rows of the 127 steps t - d a tile needs are staged in LDS.
+// The A or B operands of a product over the dimensions of row p: lane group g holds dimensions
+// 16 q + 4 g + e of step 4 q + e (the sum over k takes them in any order).
 template <int HD>
-__global__ void __launch_bounds__(64 * kTW)
-fac_tok_bwd_diag_kernel(const float* __restrict__ Q, const float* __restrict__ dO,
-                        const int64_t* __restrict__ x, int64_t V, const float* __restrict__ Ek,
-                        const float* __restrict__ Ev, int L, int H, float* __restrict__ dGb) {
-    constexpr int RS = TokLds<HD>::RS;
-    constexpr int GR = TokLds<HD>::GROWS;
-    constexpr int NF = 2 * GR * RS > (kTW - 1) * 64 * HD ? 2 * GR * RS : (kTW - 1) * 64 * HD;
-    __shared__ __align__(16) float lds[NF];
-    float* sk = lds;
-    float* sv = lds + GR * RS;
-    const int64_t D = (int64_t)H * HD;
-    const int b = blockIdx.z, h = blockIdx.y, db = blockIdx.x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int d = db * 64 + lane;
-    const bool dv = d >= 1 && d < L;
-    const int64_t* xb = x + (int64_t)b * L;
-    float dg[HD];
+__device__ inline void dim_operand(const float* p, int g, float (&v)[HD / 4]) {
 #pragma unroll
-    for (int k = 0; k < HD; ++k) dg[k] = 0.0f;
-    const int nb = (L + 63) / 64;
-    for (int tb = db; tb < nb; ++tb) {
-        const int slo = tb * 64 - db * 64 - 63;  // s = t - d spans [slo, slo + 126]
-        __syncthreads();
-        stage_tok_rows<HD>(sk, Ek, xb, V, D, h, slo, GR, L);
-        stage_tok_rows<HD>(sv, Ev, xb, V, D, h, slo, GR, L);
-        __syncthreads();
-        const int t_hi = min(tb * 64 + 64, L);
-        for (int t = tb * 64 + w; t < t_hi; t += kTW) {
-            // the walked rows come from global memory here: staging them too (104 KB of LDS)
-            // leaves one block per CU and measured slower
-            const float* q = Q + ((int64_t)b * L + t) * D + h * HD;
-            const float* go = dO + ((int64_t)b * L + t) * D + h * HD;
-            const int si = t - d - slo;
-            const bool pair = dv && t - d >= 0;
-            const float* ekr = sk + (pair ? si : 0) * RS;
-            const float* evr = sv + (pair ? si : 0) * RS;
-            float da = 0.0f;
+    for (int q = 0; q < HD / 16; ++q) {
+        const f32x4 t = load4(p, 16 * q + 4 * g);
 #pragma unroll
-            for (int k = 0; k < HD; ++k) da = __builtin_fmaf(go[k], evr[k], da);
-            da = pair ? da : 0.0f;
-#pragma unroll
-            for (int k = 0; k < HD; ++k) dg[k] = __builtin_fmaf(da * q[k], ekr[k], dg[k]);
-        }
+        for (int e = 0; e < 4; ++e) v[4 * q + e] = t[e];
     }
-    reduce_waves<HD>(dg, lds);
-    if (w == 0 && d < L) {
+}
+
+// acc[a][:] += sum_w da[w][a] y_w ⊙ g_{w,a} for the thread's TT rows and 4 dimensions: da in LDS
+// (WS floats per walked step), the rows y_w of Y from ig on, and g_{w,a} = row (first + DIR w -+ a) of
+// G: a step moves every row's distance by one.
+template <int HD, int DIR, int WS>
+__device__ inline void gate_rows(const float* da, const float* Y, const float* G, int first, int ig,
+                                 f32x4 (&acc)[HD / 16]) {
+    constexpr int TT = HD / 16;
+    f32x4 g[TT];
 #pragma unroll
-        for (int k = 0; k < HD; ++k) dGb[((int64_t)b * L + d) * D + h * HD + k] = dv ? dg[k] : 0.0f;
+    for (int a = 1; a < TT; ++a) g[a - 1] = *reinterpret_cast<const f32x4*>(G + (first - DIR * a) * HD + ig);
+    const float* gp = G + first * HD + ig;
+#pragma unroll 4
+    for (int w = 0; w < kTokB; ++w) {
+#pragma unroll
+        for (int a = TT - 1; a > 0; --a) g[a] = g[a - 1];
+        g[0] = *reinterpret_cast<const f32x4*>(gp + DIR * w * HD);
+        const f32x4 y = *reinterpret_cast<const f32x4*>(Y + w * HD + ig);
+        float d[TT];
+        if constexpr (TT == 4) {
+            const f32x4 t = *reinterpret_cast<const f32x4*>(da + w * WS);
+#pragma unroll
+            for (int a = 0; a < TT; ++a) d[a] = t[a];
+        } else {
+            const float2 t = *reinterpret_cast<const float2*>(da + w * WS);
+            d[0] = t.x; d[1] = t.y;
+        }
+#pragma unroll
+        for (int a = 0; a < TT; ++a)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[a][e] = __builtin_fmaf(d[a] * y[e], g[a][e], acc[a][e]);
+    }
+}
+
+// out[r] = sum_w dA(r, w) Y[w] ⊙ G[d], dA(r, w) = X[r] . Z[w].  ROWT: rows are steps t and the
+// walked ones s < t (dQ: X = dO, Z = e_v, Y = e_k); otherwise rows are steps s and the walked
+// ones t > s (dE_k: X = e_v, Z = dO, Y = q).
+template <int HD, bool ROWT>
+__global__ void __launch_bounds__(256, 2)
+fac_tok_gate_kernel(const float* __restrict__ Q, const float* __restrict__ dO, const int64_t* __restrict__ x,
+                    int64_t V, const float* __restrict__ Ek, const float* __restrict__ Ev,
+                    const float* __restrict__ G, int L, int H, float* __restrict__ out) {
+    constexpr int TT = HD / 16;
+    constexpr int WS = 16 + 4;  // floats per walked step of a wave's 16 rows
+    __shared__ __align__(16) float Ys[kTokB * HD], Gs[2 * kTokB * HD], dAs[4 * kTokB * WS];
+    const int64_t D = (int64_t)H * HD;
+    const int b = blockIdx.z, h = blockIdx.y, nb = gridDim.x;
+    const int rb = ROWT ? nb - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c16 = lane & 15, g = lane >> 4;
+    const int64_t* xb = x + (int64_t)b * L;
+    const int64_t slice = (int64_t)b * L * D + h * HD;
+    const TokRows go{dO + slice, nullptr, 0, D, L}, ev{Ev + h * HD, xb, V, D, L};
+    const TokRows yr = ROWT ? TokRows{Ek + h * HD, xb, V, D, L} : TokRows{Q + slice, nullptr, 0, D, L};
+    const TokRows gt{G + h * HD, nullptr, 0, D, L + 1};
+    const TokRows xr = ROWT ? go : ev, zr = ROWT ? ev : go;
+    float* da = dAs + wave * kTokB * WS;
+    const int ig = 4 * (lane % (HD / 4)), rg = TT * (lane / (HD / 4));  // 4 dimensions; TT rows of the wave
+    f32x4 acc[TT];
+#pragma unroll
+    for (int a = 0; a < TT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float xv[HD / 4];
+    dim_operand<HD>(xr.row(rb * kTokB + 16 * wave + c16), g, xv);
+    const int w_lo = ROWT ? 0 : rb, w_hi = ROWT ? rb : nb - 1;
+    for (int wb = w_lo; wb <= w_hi; ++wb) {
+        float zv[4][HD / 4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dim_operand<HD>(zr.row(wb * kTokB + 16 * j + c16), g, zv[j]);
+        __syncthreads();
+        stage_by_row<kTokB, HD, HD>(Ys, yr, wb * kTokB);
+        stage_by_row<2 * kTokB, HD, HD>(Gs, gt, (ROWT ? rb - wb : wb - rb) * kTokB - (kTokB - 1));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < HD / 4; ++k) d = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[k], zv[j][k], d, 0, 0, 0);
+            if (wb == rb || wb == nb - 1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int r = rb * kTokB + 16 * wave + 4 * g + i, w = wb * kTokB + 16 * j + c16;
+                    d[i] = (ROWT ? r > w : w > r) && w < L ? d[i] : 0.f;
+                }
+            }
+            *reinterpret_cast<f32x4*>(da + (16 * j + c16) * WS + 4 * g) = d;
+        }
+        __syncthreads();
+        // distance of row r and walked step w: row r - w + 63 of the staged ones (ROWT), w - r + 63
+        const int r0 = 16 * wave + rg;
+        if (ROWT) gate_rows<HD, -1, WS>(da + rg, Ys, Gs, r0 + kTokB - 1, ig, acc);
+        else gate_rows<HD, 1, WS>(da + rg, Ys, Gs, kTokB - 1 - r0, ig, acc);
+    }
+#pragma unroll
+    for (int a = 0; a < TT; ++a) {
+        const int r = rb * kTokB + 16 * wave + rg + a;
+        if (r >= L) continue;
+        const bool ok = ROWT || ev.row(r);
+        *reinterpret_cast<f32x4u*>(out + slice + (int64_t)r * D + ig) = ok ? acc[a] : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+// Rows are distances d, walked steps t: dGb[b,d,h,:] = sum_t (dO_t . e_v[x_{t-d}]) q_t ⊙
+// e_k[x_{t-d}] for d in [1, L); row 0 is zero.  The steps s = t - d of a tile span 127 rows; the
+// products dO_t . e_v[x_s] of a wave's 16 steps t fall on 79 of them, five column tiles.
+template <int HD>
+__global__ void __launch_bounds__(256, 2)
+fac_tok_dist_kernel(const float* __restrict__ Q, const float* __restrict__ dO, const int64_t* __restrict__ x,
+                    int64_t V, const float* __restrict__ Ek, const float* __restrict__ Ev, int L, int H,
+                    float* __restrict__ dGb) {
+    constexpr int TT = HD / 16;
+    constexpr int WS = kTokB + 4;
+    __shared__ __align__(16) float Qs[kTokB * HD], Es[2 * kTokB * HD], dAs[kTokB * WS];
+    const int64_t D = (int64_t)H * HD;
+    const int b = blockIdx.z, h = blockIdx.y, nb = gridDim.x, db = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c16 = lane & 15, g = lane >> 4;
+    const int64_t* xb = x + (int64_t)b * L;
+    const int64_t slice = (int64_t)b * L * D + h * HD;
+    const TokRows qr{Q + slice, nullptr, 0, D, L}, go{dO + slice, nullptr, 0, D, L};
+    const TokRows ek{Ek + h * HD, xb, V, D, L}, ev{Ev + h * HD, xb, V, D, L};
+    const int ig = 4 * (lane % (HD / 4)), rg = TT * (lane / (HD / 4));
+    f32x4 acc[TT];
+#pragma unroll
+    for (int a = 0; a < TT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tb = db; tb < nb; ++tb) {
+        const int slo = (tb - db) * kTokB - (kTokB - 1);
+        float xv[HD / 4], zv[5][HD / 4];
+        dim_operand<HD>(go.row(tb * kTokB + 16 * wave + c16), g, xv);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) dim_operand<HD>(ev.row(slo + 16 * (wave + j) + c16), g, zv[j]);
+        __syncthreads();
+        stage_by_row<kTokB, HD, HD>(Qs, qr, tb * kTokB);
+        stage_by_row<2 * kTokB, HD, HD>(Es, ek, slo);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < HD / 4; ++k) v = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[k], zv[j][k], v, 0, 0, 0);
+            const int si = 16 * (wave + j) + c16;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * wave + 4 * g + i, d = t + kTokB - 1 - si;
+                if (d >= 0 && d < kTokB) dAs[t * WS + d] = slo + si >= 0 && db + d > 0 && tb * kTokB + t < L ? v[i] : 0.f;
+            }
+        }
+        __syncthreads();
+        const int d0 = 16 * wave + rg;
+        gate_rows<HD, 1, WS>(dAs + d0, Qs, Es, kTokB - 1 - d0, ig, acc);
+    }
+#pragma unroll
+    for (int a = 0; a < TT; ++a) {
+        const int d = db * kTokB + 16 * wave + rg + a;
+        if (d < L) *reinterpret_cast<f32x4u*>(dGb + slice + (int64_t)d * D + ig) = acc[a];
     }
 }
 
@@ -754,11 +776,11 @@ extern "C" int mb_factored_tok_fwd(const float* Q, const int64_t* x, int64_t V, 
     if (B == 0 || L == 0) return MB_OK;
     MB_REQUIRE(Q && x && E_k && E_v && G && O, "mb_factored_tok_fwd: null pointer argument");
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((L + 63) / 64, H, B), blk(64 * kTW);
+    const dim3 grid((L + kTokB - 1) / kTokB, H, B), blk(256);
     if (hd == 64)
-        hipLaunchKernelGGL(fac_tok_fwd_kernel<64>, grid, blk, 0, st, Q, x, V, E_k, E_v, G, L, H, O);
+        hipLaunchKernelGGL((fac_tok_pair_kernel<64, true>), grid, blk, 0, st, Q, nullptr, x, V, E_k, E_v, G, L, H, O);
     else
-        hipLaunchKernelGGL(fac_tok_fwd_kernel<32>, grid, blk, 0, st, Q, x, V, E_k, E_v, G, L, H, O);
+        hipLaunchKernelGGL((fac_tok_pair_kernel<32, true>), grid, blk, 0, st, Q, nullptr, x, V, E_k, E_v, G, L, H, O);
     return check_launch("mb_factored_tok_fwd");
 }
 
@@ -772,17 +794,16 @@ extern "C" int mb_factored_tok_bwd(const float* Q, const float* dO, const int64_
     MB_REQUIRE(Q && dO && x && E_k && E_v && G && dQ && dEk_tok && dEv_tok && dG_b,
                "mb_factored_tok_bwd: null pointer argument");
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((L + 63) / 64, H, B), blk(64 * kTW);
-#define MB_FAC_BWD(HDV)                                                                           \
-    do {                                                                                          \
-        hipLaunchKernelGGL(fac_tok_bwd_row_kernel<HDV>, grid, blk, 0, st, dO, x, V, E_k, E_v, G, L, \
-                           H, dQ);                                                                \
-        hipLaunchKernelGGL((fac_tok_bwd_col_kernel<HDV, true>), grid, blk, 0, st, Q, dO, x, V, E_k, \
-                           E_v, G, L, H, dEk_tok);                                                \
-        hipLaunchKernelGGL((fac_tok_bwd_col_kernel<HDV, false>), grid, blk, 0, st, Q, dO, x, V,     \
-                           E_k, E_v, G, L, H, dEv_tok);                                           \
-        hipLaunchKernelGGL(fac_tok_bwd_diag_kernel<HDV>, grid, blk, 0, st, Q, dO, x, V, E_k, E_v, L, \
-                           H, dG_b);                                                              \
+    const dim3 grid((L + kTokB - 1) / kTokB, H, B), blk(256);
+#define MB_FAC_BWD(HDV)                                                                            \
+    do {                                                                                           \
+        hipLaunchKernelGGL((fac_tok_gate_kernel<HDV, true>), grid, blk, 0, st, Q, dO, x, V, E_k, E_v, G, L, H, \
+                           dQ);                                                                    \
+        hipLaunchKernelGGL((fac_tok_gate_kernel<HDV, false>), grid, blk, 0, st, Q, dO, x, V, E_k, E_v, G, L, H, \
+                           dEk_tok);                                                               \
+        hipLaunchKernelGGL((fac_tok_pair_kernel<HDV, false>), grid, blk, 0, st, Q, dO, x, V, E_k, E_v, G, L, H, \
+                           dEv_tok);                                                               \
+        hipLaunchKernelGGL(fac_tok_dist_kernel<HDV>, grid, blk, 0, st, Q, dO, x, V, E_k, E_v, L, H, dG_b); \
     } while (0)
     if (hd == 64) MB_FAC_BWD(64);
     else MB_FAC_BWD(32);

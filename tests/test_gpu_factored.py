@@ -82,6 +82,29 @@ def test_gpu_factored_model_shape():
     assert max(errs.values()) < TOL, errs
 
 
+@pytest.mark.parametrize("L,hd", [(64, 64), (129, 32), (191, 64), (193, 32)])
+def test_gpu_factored_token_blocks(L, hd):
+    # the last block's partial rows and distances; ids outside [0, V) read as zero rows; and Q
+    # at an address that is only 4-byte aligned
+    from mathbrain.factored_ema import factored_ema_forward
+    (Q, x, Ek, Ev, rhos, W, H), _ = make(2, L, 40, 3, hd, 8, 0, seed=L, cbase=False)
+    V, D = Ek.shape
+    bad = torch.rand(x.shape, generator=torch.Generator().manual_seed(L)) < 0.1
+    zero = torch.zeros(1, D, dtype=torch.float64)
+    leaves = [t.clone().requires_grad_(True) for t in (Q, torch.cat([Ek, zero]), torch.cat([Ev, zero]), W)]
+    want = of.closed_form(leaves[0], torch.where(bad, V, x), leaves[1], leaves[2], rhos, leaves[3], H)
+    dO = torch.randn(want.shape, generator=torch.Generator().manual_seed(1), dtype=torch.float64)
+    want.backward(dO)
+    f = lambda t: t.to(torch.float32).cuda()
+    shifted = torch.empty(Q.numel() + 1, device="cuda")[1:].view(Q.shape).copy_(f(Q))
+    dl = [t.requires_grad_(True) for t in (shifted, f(Ek), f(Ev), f(W))]
+    ids = torch.where(bad, torch.where(x % 2 == 0, -3, V + 5), x).cuda()
+    got = factored_ema_forward(dl[0], ids, dl[1], dl[2], f(rhos), dl[3], H)
+    got.backward(f(dO))
+    errs = [rel(got, want)] + [rel(a.grad, b.grad[:len(a)]) for a, b in zip(dl, leaves)]
+    assert max(errs) < TOL, errs
+
+
 def test_gpu_factored_matches_loop_restatement():
     # the step-by-step restatement of factored_ema.py:22-96 (not only its closed form)
     from mathbrain.factored_ema import factored_ema_forward
