@@ -179,196 +179,300 @@ fac_apply_kernel(const float* __restrict__ M, const float* __restrict__ w, int64
 // The state contractions are plain GEMMs per rate.  These forms run them on the bf16 matrix
 // cores with every fp32 operand split into bf16 hi + lo parts and three products
 // (hi*hi + hi*lo + lo*hi, fp32 accumulation), which keeps about 2^-16 relative error per
-// product.  Operand layout of v_mfma_f32_16x16x16_bf16: A[row = lane%16][k = 4 (lane/16) + e],
-// B[k = 4 (lane/16) + e][col = lane%16], D[row = 4 (lane/16) + i][col = lane%16].
+// product.  Operand layout of v_mfma_f32_16x16x32_bf16: A[row = lane%16][k = 8 (lane/16) + e],
+// B[k = 8 (lane/16) + e][col = lane%16], D[row = 4 (lane/16) + i][col = lane%16].
+// Bound: the matrix cores, provided that an operand is split once per workgroup and not once per
+// wave, and that the loads run a tile ahead.  B56 T512 H8 N64 with a history of 4 096 tokens,
+// forward + backward: fac_outer 3.00 -> 1.70 ms, fac_apply 5.34 -> 3.17 ms against four waves
+// that each split their own tiles, unprefetched, for the half-rate 16x16x16 form.
 
-__device__ inline void split_bf16x4(const float (&v)[4], bf16x4& hi, bf16x4& lo) {
+constexpr int kStateDim = 64;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ inline void split_bf16x8(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < 8; ++e) {
         const __bf16 t = (__bf16)v[e];
         hi[e] = t;
         lo[e] = (__bf16)(v[e] - (float)t);
     }
 }
 
-__device__ inline f32x4 mfma3(bf16x4 ah, bf16x4 al, bf16x4 bh, bf16x4 bl, f32x4 c) {
-    c = mfma16x16x16(ah, bh, c);
-    c = mfma16x16x16(ah, bl, c);
-    return mfma16x16x16(al, bh, c);
+__device__ inline f32x4 mfma3(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl, f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c, 0, 0, 0);
 }
 
-// fac_apply_kernel for hd = 64: block (64 rows, h, b); wave w owns outputs [16w, 16w + 16)
-// of the 64 rows (4 row tiles); the Y rows are split once, each rate's M_n tile per rate.
+// Workgroup id -> (block r < nr, head bh = b H + h).  The nr blocks of a head read the same
+// tiles: where the heads divide among the 8 XCDs (ids go to them round-robin), they share one
+// XCD's L2.
+struct HeadBlock {
+    int r, bh;
+};
+__device__ inline HeadBlock head_block(int id, int nr, int heads) {
+    if (heads % 8) return HeadBlock{id % nr, id / nr};
+    const int k = id >> 3;
+    return HeadBlock{k % nr, (k / nr) * 8 + (id & 7)};
+}
+
+// fac_apply_kernel for hd = 64: 128 rows of a head, 8 waves of 32 rows x 32 outputs.  The Y rows
+// are split once; a rate's scaled and oriented M_n is split once for the workgroup, into one of
+// two LDS buffers, while the next rate's is on its way.
+constexpr int kStateRows = 128;
+
 template <bool TRANS>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512, 4)
 fac_apply_mfma_kernel(const float* __restrict__ M, const float* __restrict__ w, int64_t ldw,
                       const float* __restrict__ Y, const int64_t* __restrict__ yrow, int64_t ld,
                       int64_t nrows, const float* __restrict__ alpha, int64_t as_b, int64_t as_r,
-                      int64_t as_n, int R, int H, int N, float* __restrict__ out, int64_t ldo,
+                      int64_t as_n, int B, int R, int H, int N, float* __restrict__ out, int64_t ldo,
                       int accumulate) {
-    constexpr int HD = 64;
-    constexpr int AN = 64;
-    __shared__ float As[64 * AN];
-    const int b = blockIdx.z, h = blockIdx.y;
-    const int r0 = blockIdx.x * 64;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    constexpr int HD = kStateDim;
+    constexpr int AN = 64;               // rates whose alphas are staged at once
+    constexpr int AS = kStateRows + 4;   // floats per rate
+    constexpr int MS = HD + 8;           // bf16 per output column: 16-byte reads on all banks
+    __shared__ __align__(16) float As[AN * AS];
+    __shared__ __align__(16) __bf16 Mt[2][2][HD * MS];  // [buffer][hi, lo][output][k]
+    const int nr = (R + kStateRows - 1) / kStateRows;
+    const HeadBlock hb = head_block(blockIdx.x, nr, B * H);
+    const int b = hb.bh / H, h = hb.bh % H;
+    const int r0 = hb.r * kStateRows;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c16 = lane & 15, g = lane >> 4;
-    bf16x4 ahi[4][4], alo[4][4];
+    const int rw = 32 * (wave & 3), cw = 32 * (wave >> 2);
+    bf16x8 ahi[2][2], alo[2][2];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int r = r0 + 16 * rt + c16;
+    for (int rt = 0; rt < 2; ++rt) {
+        const int r = r0 + rw + 16 * rt + c16;
         const int64_t ry = r < R ? clamp_row(yrow, (int64_t)b * R + r, nrows) : -1;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            float v[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int ks = 0; ks < 2; ++ks) {
+            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (ry >= 0) {
-                const float4 q = *reinterpret_cast<const float4*>(Y + ry * ld + h * HD + 16 * kt + 4 * g);
-                v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+                const float* p = Y + ry * ld + h * HD + 32 * ks + 8 * g;
+                const f32x4u q0 = *reinterpret_cast<const f32x4u*>(p), q1 = *reinterpret_cast<const f32x4u*>(p + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { v[e] = q0[e]; v[4 + e] = q1[e]; }
             }
-            split_bf16x4(v, ahi[rt][kt], alo[rt][kt]);
+            split_bf16x8(v, ahi[rt][ks], alo[rt][ks]);
         }
     }
-    f32x4 acc[4];
+    // this thread's part of a tile: output column mo, k = mk .. mk + 7
+    const int mo = TRANS ? lane : tid >> 3, mk = 8 * (TRANS ? wave : tid & 7);
+    const float* Mb = M + (int64_t)hb.bh * N * HD * HD;
+    const float* wh = w ? w + h * HD : nullptr;
+    float m[8], ms[8];
+    auto load_tile = [&](int n) {
+        const float* Mn = Mb + (int64_t)n * HD * HD;
+        if (!TRANS) {  // B[k][o] = w[n, o] M_n[o][k]
+            const f32x4 q0 = *reinterpret_cast<const f32x4*>(Mn + mo * HD + mk);
+            const f32x4 q1 = *reinterpret_cast<const f32x4*>(Mn + mo * HD + mk + 4);
+            ms[0] = wh ? wh[n * ldw + mo] : 1.0f;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int o = 16 * wv + c16;
-    const float* Mb = M + ((int64_t)b * H + h) * N * HD * HD;
+            for (int e = 0; e < 4; ++e) { m[e] = q0[e]; m[4 + e] = q1[e]; }
+        } else {       // B[k][o] = w[n, k] M_n[k][o]
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                m[e] = Mn[(mk + e) * HD + mo];
+                ms[e] = wh ? wh[n * ldw + mk + e] : 1.0f;
+            }
+        }
+    };
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    load_tile(0);
     for (int n = 0; n < N; ++n) {
         if (n % AN == 0) {
             __syncthreads();
-            for (int e = tid; e < 64 * AN; e += 256) {
-                const int rr = e / AN, nn = n + e % AN;
-                As[e] = (r0 + rr < R && nn < N)
-                            ? alpha[b * as_b + (int64_t)(r0 + rr) * as_r + nn * as_n] : 0.0f;
+            for (int e = tid; e < kStateRows * AN; e += 512) {
+                const int rr = e / AN, nn = e % AN;
+                As[nn * AS + rr] = (r0 + rr < R && n + nn < N)
+                                       ? alpha[b * as_b + (int64_t)(r0 + rr) * as_r + (n + nn) * as_n] : 0.0f;
             }
-            __syncthreads();
         }
-        const float* Mn = Mb + (int64_t)n * HD * HD;
-        bf16x4 bhi[4], blo[4];
+        __bf16* buf = Mt[n & 1][0];
+        {
+            float v[8];
+            bf16x8 hi, lo;
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            float v[4];
-            if (!TRANS) {  // B[k][o] = w[n, o] M_n[o][k]
-                const float4 q = *reinterpret_cast<const float4*>(Mn + o * HD + 16 * kt + 4 * g);
-                const float ws = w ? w[n * ldw + h * HD + o] : 1.0f;
-                v[0] = q.x * ws; v[1] = q.y * ws; v[2] = q.z * ws; v[3] = q.w * ws;
-            } else {       // B[k][o] = w[n, k] M_n[k][o]
+            for (int e = 0; e < 8; ++e) v[e] = m[e] * ms[TRANS ? e : 0];
+            split_bf16x8(v, hi, lo);
+            *reinterpret_cast<bf16x8*>(buf + mo * MS + mk) = hi;
+            *reinterpret_cast<bf16x8*>(buf + HD * MS + mo * MS + mk) = lo;
+        }
+        if (n + 1 < N) load_tile(n + 1);
+        __syncthreads();
+        f32x4 s[2][2];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int k = 16 * kt + 4 * g + e;
-                    v[e] = Mn[k * HD + o] * (w ? w[n * ldw + h * HD + k] : 1.0f);
-                }
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) s[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const __bf16* p = buf + (cw + 16 * ct + c16) * MS + 32 * ks + 8 * g;
+                const bf16x8 bh = *reinterpret_cast<const bf16x8*>(p);
+                const bf16x8 bl = *reinterpret_cast<const bf16x8*>(p + HD * MS);
+#pragma unroll
+                for (int rt = 0; rt < 2; ++rt) s[rt][ct] = mfma3(ahi[rt][ks], alo[rt][ks], bh, bl, s[rt][ct]);
             }
-            split_bf16x4(v, bhi[kt], blo[kt]);
-        }
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+        for (int rt = 0; rt < 2; ++rt) {
+            const f32x4 al = *reinterpret_cast<const f32x4*>(As + (n % AN) * AS + rw + 16 * rt + 4 * g);
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) sacc = mfma3(ahi[rt][kt], alo[rt][kt], bhi[kt], blo[kt], sacc);
+            for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[rt][i] = __builtin_fmaf(As[(16 * rt + 4 * g + i) * AN + n % AN], sacc[i], acc[rt][i]);
+                for (int i = 0; i < 4; ++i) acc[rt][ct][i] = __builtin_fmaf(al[i], s[rt][ct][i], acc[rt][ct][i]);
         }
     }
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = r0 + 16 * rt + 4 * g + i;
+            const int r = r0 + rw + 16 * rt + 4 * g + i;
             if (r >= R) continue;
-            float* dst = out + ((int64_t)b * R + r) * ldo + h * HD + o;
-            *dst = accumulate ? *dst + acc[rt][i] : acc[rt][i];
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) {
+                float* dst = out + ((int64_t)b * R + r) * ldo + h * HD + cw + 16 * ct + c16;
+                *dst = accumulate ? *dst + acc[rt][ct][i] : acc[rt][ct][i];
+            }
         }
 }
 
-// fac_outer_kernel for hd = 64: block (4 rates, h, b), wave w = rate 4 blockIdx.x + w, the
-// whole 64 x 64 output of its rate in 16 tiles.  The walked rows come in blocks of 32 (two
-// MFMA k steps), staged in LDS once for the four rates: they share the X and Y rows and
-// differ only in the weights alpha.
+// fac_outer_kernel for hd = 64: 8 rates of a head, two per wave, each the whole 64 x 64 output of
+// its rate in 16 tiles.  The walked rows come in blocks of 32 (one MFMA k step), staged with the
+// row as the fast index: X in fp32 (each rate weights it before the split), Y split.  Two rates
+// to a wave halve the LDS reads per product (one rate: 18 of 16 bytes per 48; two: 20 per 96).
 constexpr int kOuterRows = 32;
+constexpr int kOuterRates = 8;
 
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 fac_outer_mfma_kernel(const float* __restrict__ X, const int64_t* __restrict__ xrow,
                       const float* __restrict__ Y, const int64_t* __restrict__ yrow, int64_t ld,
                       int64_t nrows, const float* __restrict__ alpha, int64_t as_b, int64_t as_r,
-                      int64_t as_n, int R, int H, int N, float* __restrict__ out) {
-    constexpr int HD = 64;
-    constexpr int RS = HD + 4;
-    __shared__ __align__(16) float Xs[kOuterRows * RS];
-    __shared__ __align__(16) float Ys[kOuterRows * RS];
-    const int b = blockIdx.z, h = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int n = blockIdx.x * 4 + (tid >> 6);
+                      int64_t as_n, int B, int R, int H, int N, float* __restrict__ out) {
+    constexpr int HD = kStateDim;
+    constexpr int XS = kOuterRows + 4;  // floats per dimension
+    constexpr int YS = kOuterRows + 8;  // bf16 per dimension
+    __shared__ __align__(16) float Xs[2][HD * XS], As[2][kOuterRates * XS];
+    __shared__ __align__(16) __bf16 Ys[2][2][HD * YS];  // [buffer][hi, lo]
+    const int nr = (N + kOuterRates - 1) / kOuterRates;
+    const HeadBlock hb = head_block(blockIdx.x, nr, B * H);
+    const int b = hb.bh / H, h = hb.bh % H;
+    const int n0 = hb.r * kOuterRates;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c16 = lane & 15, g = lane >> 4;
-    const bool nv = n < N;
-    f32x4 acc[4][4];
+    // staged by this thread: rows 2 sp, 2 sp + 1 of dimensions sc .. sc + 3, and one alpha
+    const int sp = (tid >> 2) & 15, sc = 4 * ((tid & 3) + 4 * wave);
+    const int an = tid & (kOuterRates - 1), ar = tid / kOuterRates;
+    int64_t rx[2], ry[2];
+    f32x4 vx[2], vy[2];
+    float va;
+    auto load_ids = [&](int k0) {
 #pragma unroll
-    for (int it = 0; it < 4; ++it)
+        for (int e = 0; e < 2; ++e) {
+            const int r = k0 + 2 * sp + e;
+            const int64_t ex = (int64_t)b * R + r;
+            rx[e] = r < R ? clamp_row(xrow, ex, nrows) : -1;
+            ry[e] = r < R ? clamp_row(yrow, ex, nrows) : -1;
+        }
+    };
+    auto load_rows = [&](int k0) {
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt) acc[it][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < R; k0 += kOuterRows) {
-        __syncthreads();
-        // stage the block's rows: thread tid copies float4 (tid % 16) of row tid / 16 of X
-        // and of Y (rows of zero weight for every rate are staged as zeros)
-        for (int e = tid; e < kOuterRows * (HD / 4); e += 256) {
-            const int rr = e / (HD / 4), c = e % (HD / 4);
-            const int r = k0 + rr;
-            float4 vx = make_float4(0.f, 0.f, 0.f, 0.f), vy = vx;
-            if (r < R) {
-                const int64_t ex = (int64_t)b * R + r;
-                const int64_t rx = clamp_row(xrow, ex, nrows), ry = clamp_row(yrow, ex, nrows);
-                if (rx >= 0 && ry >= 0) {
-                    vx = *reinterpret_cast<const float4*>(X + rx * ld + h * HD + 4 * c);
-                    vy = *reinterpret_cast<const float4*>(Y + ry * ld + h * HD + 4 * c);
-                }
+        for (int e = 0; e < 2; ++e) {
+            const bool ok = rx[e] >= 0 && ry[e] >= 0;
+            vx[e] = ok ? f32x4(*reinterpret_cast<const f32x4u*>(X + rx[e] * ld + h * HD + sc)) : f32x4{0.f, 0.f, 0.f, 0.f};
+            vy[e] = ok ? f32x4(*reinterpret_cast<const f32x4u*>(Y + ry[e] * ld + h * HD + sc)) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int r = k0 + ar, n = n0 + an;
+        va = r < R && n < N ? alpha[b * as_b + (int64_t)r * as_r + n * as_n] : 0.0f;
+    };
+    f32x4 acc[2][4][4];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int it = 0; it < 4; ++it)
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) acc[q][it][jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    load_ids(0);
+    load_rows(0);
+    load_ids(kOuterRows);
+    for (int k0 = 0, buf = 0; k0 < R; k0 += kOuterRows, buf ^= 1) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            *reinterpret_cast<float2*>(Xs[buf] + (sc + e) * XS + 2 * sp) = make_float2(vx[0][e], vx[1][e]);
+            __bf16 hi[2], lo[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                hi[q] = (__bf16)vy[q][e];
+                lo[q] = (__bf16)(vy[q][e] - (float)hi[q]);
             }
-            *reinterpret_cast<float4*>(Xs + rr * RS + 4 * c) = vx;
-            *reinterpret_cast<float4*>(Ys + rr * RS + 4 * c) = vy;
+            typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+            *reinterpret_cast<bf16x2*>(Ys[buf][0] + (sc + e) * YS + 2 * sp) = bf16x2{hi[0], hi[1]};
+            *reinterpret_cast<bf16x2*>(Ys[buf][1] + (sc + e) * YS + 2 * sp) = bf16x2{lo[0], lo[1]};
+        }
+        As[buf][an * XS + ar] = va;
+        if (k0 + kOuterRows < R) {
+            load_rows(k0 + kOuterRows);
+            load_ids(k0 + 2 * kOuterRows);
         }
         __syncthreads();
+        float al[2][8];
+        bool any = false;
 #pragma unroll
-        for (int ks = 0; ks < kOuterRows / 16; ++ks) {
-            float al[4];
-            bool any = false;
+        for (int q = 0; q < 2; ++q) {
+            const float* p = As[buf] + (2 * wave + q) * XS + 8 * g;
+            const f32x4 t0 = *reinterpret_cast<const f32x4*>(p), t1 = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int r = k0 + 16 * ks + 4 * g + e;
-                al[e] = (nv && r < R) ? alpha[b * as_b + (int64_t)r * as_r + n * as_n] : 0.0f;
-                any = any || al[e] != 0.0f;
+                al[q][e] = t0[e];
+                al[q][4 + e] = t1[e];
+                any = any || t0[e] != 0.0f || t1[e] != 0.0f;
             }
-            if (!__any(any)) continue;
-            const float* xr = Xs + (16 * ks + 4 * g) * RS;
-            const float* yr = Ys + (16 * ks + 4 * g) * RS;
-            bf16x4 ahi[4], alo[4], bhi[4], blo[4];
+        }
+        if (!__any(any)) continue;
+        bf16x8 bh[4], bl[4];
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                float v[4];
+        for (int jt = 0; jt < 4; ++jt) {
+            bh[jt] = *reinterpret_cast<const bf16x8*>(Ys[buf][0] + (16 * jt + c16) * YS + 8 * g);
+            bl[jt] = *reinterpret_cast<const bf16x8*>(Ys[buf][1] + (16 * jt + c16) * YS + 8 * g);
+        }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = al[e] * xr[e * RS + 16 * it + c16];
-                split_bf16x4(v, ahi[it], alo[it]);
+        for (int it = 0; it < 4; ++it) {
+            const float* p = Xs[buf] + (16 * it + c16) * XS + 8 * g;
+            const f32x4 t0 = *reinterpret_cast<const f32x4*>(p), t1 = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float v[8];
+                bf16x8 ah, alo;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = al[q][e] * t0[e];
+                    v[4 + e] = al[q][4 + e] * t1[e];
+                }
+                split_bf16x8(v, ah, alo);
+#pragma unroll
+                for (int jt = 0; jt < 4; ++jt) acc[q][it][jt] = mfma3(ah, alo, bh[jt], bl[jt], acc[q][it][jt]);
             }
-#pragma unroll
-            for (int jt = 0; jt < 4; ++jt) {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = yr[e * RS + 16 * jt + c16];
-                split_bf16x4(v, bhi[jt], blo[jt]);
-            }
-#pragma unroll
-            for (int it = 0; it < 4; ++it)
-#pragma unroll
-                for (int jt = 0; jt < 4; ++jt) acc[it][jt] = mfma3(ahi[it], alo[it], bhi[jt], blo[jt], acc[it][jt]);
         }
     }
-    if (!nv) return;
-    float* o = out + (((int64_t)b * H + h) * N + n) * HD * HD;
 #pragma unroll
-    for (int it = 0; it < 4; ++it)
+    for (int q = 0; q < 2; ++q) {
+        const int n = n0 + 2 * wave + q;
+        if (n >= N) continue;
+        float* o = out + ((int64_t)hb.bh * N + n) * HD * HD;
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt)
+        for (int it = 0; it < 4; ++it)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[(16 * it + 4 * g + i) * HD + 16 * jt + c16] = acc[it][jt][i];
+            for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[(16 * it + 4 * g + i) * HD + 16 * jt + c16] = acc[q][it][jt][i];
+    }
 }
 
 __device__ inline bool tok_ok(int64_t v, int64_t V) { return v >= 0 && v < V; }
@@ -397,7 +501,6 @@ __device__ inline bool tok_ok(int64_t v, int64_t V) { return v >= 0 && v < V; }
 // dE_k 0.82, dG 1.08); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.61 ms.
 
 constexpr int kTokB = 64;  // steps per block
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // Rows of one head: of a [L, D] slice (ids NULL), or E[x[r]] of a table; rows outside [0, L) and
 // ids outside [0, V) read as zeros.
@@ -727,8 +830,10 @@ extern "C" int mb_factored_outer(const float* X, const int64_t* xrow, const floa
     hipStream_t st = (hipStream_t)stream;
     const dim3 blk(256);
     if (hd == 64) {
-        hipLaunchKernelGGL(fac_outer_mfma_kernel, dim3((N + 3) / 4, H, B), blk, 0, st, X, xrow, Y,
-                           yrow, ld, nrows, alpha, as_b, as_r, as_n, R, H, N, out);
+        const int64_t grid = (int64_t)B * H * ((N + kOuterRates - 1) / kOuterRates);
+        MB_REQUIRE(grid <= INT32_MAX, "mb_factored_outer: B=%d H=%d N=%d too large", B, H, N);
+        hipLaunchKernelGGL(fac_outer_mfma_kernel, dim3((unsigned)grid), blk, 0, st, X, xrow, Y, yrow, ld, nrows,
+                           alpha, as_b, as_r, as_n, B, R, H, N, out);
     } else {
         hipLaunchKernelGGL(fac_outer_kernel<32>, dim3((N + 7) / 8, H, B), blk, 0, st, X, xrow, Y,
                            yrow, ld, nrows, alpha, as_b, as_r, as_n, R, H, N, out);
@@ -754,13 +859,14 @@ extern "C" int mb_factored_apply(const float* M, const float* w, int64_t ldw, co
     hipLaunchKernelGGL((fac_apply_kernel<HDV, TR>), grid, blk, 0, st, M, w, ldw, Y, yrow, ld, nrows, \
                        alpha, as_b, as_r, as_n, R, H, N, out, ldo, accumulate)
     if (hd == 64) {
-        const dim3 g64((R + 63) / 64, H, B);
+        const int64_t g64 = (int64_t)B * H * ((R + kStateRows - 1) / kStateRows);
+        MB_REQUIRE(g64 <= INT32_MAX, "mb_factored_apply: B=%d H=%d R=%d too large", B, H, R);
         if (transpose)
-            hipLaunchKernelGGL(fac_apply_mfma_kernel<true>, g64, blk, 0, st, M, w, ldw, Y, yrow, ld,
-                               nrows, alpha, as_b, as_r, as_n, R, H, N, out, ldo, accumulate);
+            hipLaunchKernelGGL(fac_apply_mfma_kernel<true>, dim3((unsigned)g64), dim3(512), 0, st, M, w, ldw, Y, yrow,
+                               ld, nrows, alpha, as_b, as_r, as_n, B, R, H, N, out, ldo, accumulate);
         else
-            hipLaunchKernelGGL(fac_apply_mfma_kernel<false>, g64, blk, 0, st, M, w, ldw, Y, yrow, ld,
-                               nrows, alpha, as_b, as_r, as_n, R, H, N, out, ldo, accumulate);
+            hipLaunchKernelGGL(fac_apply_mfma_kernel<false>, dim3((unsigned)g64), dim3(512), 0, st, M, w, ldw, Y, yrow,
+                               ld, nrows, alpha, as_b, as_r, as_n, B, R, H, N, out, ldo, accumulate);
     } else {
         if (transpose) MB_FAC_APPLY(32, true); else MB_FAC_APPLY(32, false);
     }

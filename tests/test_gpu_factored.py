@@ -82,6 +82,15 @@ def test_gpu_factored_model_shape():
     assert max(errs.values()) < TOL, errs
 
 
+@pytest.mark.parametrize("B,L,H,N,K", [(1, 129, 8, 65, 33), (3, 127, 2, 9, 32), (2, 128, 4, 8, 161), (1, 5, 1, 7, 1)])
+def test_gpu_factored_state_tiles(B, L, H, N, K):
+    # the state kernels' edges at head_dim 64: 128 rows, 32 walked rows, 8 and 64 rates, and
+    # heads that divide among the XCDs or do not
+    args, kw = make(B, L, 300, H, 64, N, K, seed=L)
+    errs = run_both(args, kw)
+    assert max(errs.values()) < TOL, errs
+
+
 @pytest.mark.parametrize("L,hd", [(64, 64), (129, 32), (191, 64), (193, 32)])
 def test_gpu_factored_token_blocks(L, hd):
     # the last block's partial rows and distances; ids outside [0, V) read as zero rows; and Q
