@@ -497,54 +497,76 @@ __device__ inline bool tok_ok(int64_t v, int64_t V) { return v >= 0 && v < V; }
 // dimension (A in the forward and for dE_v, dQ, dE_k and dG: 10 in all), and next to it the LDS
 // reads, 3 or 4 of 16 bytes per 32 operations.  Lanes as steps with whole rows in registers
 // instead read G from LDS for every pair and dimension, and the other rows once per wave.
-// B56 T512 H8 head_dim 64, forward + backward: 9.4 -> 4.25 ms (o 0.78, dE_v 0.74, dQ 0.84,
-// dE_k 0.82, dG 1.08); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.61 ms.
+// B56 T512 H8 head_dim 64, forward + backward: 9.4 -> 3.9 ms (o 0.78, dE_v 0.67, dQ 0.78,
+// dE_k 0.68, dG 1.00); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.61 ms.
 
 constexpr int kTokB = 64;  // steps per block
 
 // Rows of one head: of a [L, D] slice (ids NULL), or E[x[r]] of a table; rows outside [0, L) and
-// ids outside [0, V) read as zeros.
+// ids outside [0, V) read as zeros.  Their address is another row's and the zeros are selected
+// after the load: a load under a condition is issued alone, and its id before it (the kernels of
+// a forward and backward at B56 T512 took 4.34 ms so, 3.91 with a tile's loads in flight together).
 struct TokRows {
     const float* p;
     const int64_t* ids;
     int64_t V, D;
     int L;
-    __device__ inline const float* row(int r) const {
-        if (r < 0 || r >= L) return nullptr;
-        if (!ids) return p + r * D;
-        const int64_t v = ids[r];
-        return tok_ok(v, V) ? p + v * D : nullptr;
+    __device__ inline const float* row(int r, bool& ok) const {
+        ok = r >= 0 && r < L;
+        int64_t v = min(max(r, 0), L - 1);
+        if (ids) {
+            v = ids[v];
+            ok = ok && tok_ok(v, V);
+            v = tok_ok(v, V) ? v : 0;
+        }
+        return p + v * D;
     }
 };
 
-__device__ inline f32x4 load4(const float* p, int c) {
-    return p ? f32x4(*reinterpret_cast<const f32x4u*>(p + c)) : f32x4{0.f, 0.f, 0.f, 0.f};
+__device__ inline f32x4 load4(const float* p, int c, bool ok) {
+    const f32x4 v = *reinterpret_cast<const f32x4u*>(p + c);
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = ok ? v[e] : 0.f;
+    return o;
 }
 
 // dst[k][r] = rows lo + r, dimensions k0 + k, for ROWS x KC; RS floats per dimension.  Four lanes
 // on 64 bytes of a row and 16 rows per wave: the transposed writes use every bank twice.
 template <int ROWS, int KC, int RS>
 __device__ inline void stage_by_dim(float* dst, const TokRows& src, int lo, int k0) {
+    constexpr int NV = (ROWS / 16) * (KC / 16) / 4;
     const int cl = threadIdx.x & 3, rl = (threadIdx.x >> 2) & 15, wave = threadIdx.x >> 6;
+    f32x4 v[NV];
 #pragma unroll
-    for (int rest = 0; rest < (ROWS / 16) * (KC / 16); rest += 4) {
-        const int r = ((rest + wave) % (ROWS / 16)) * 16 + rl;
-        const int c = ((rest + wave) / (ROWS / 16)) * 16 + 4 * cl;
-        const f32x4 v = load4(src.row(lo + r), k0 + c);
+    for (int q = 0; q < NV; ++q) {
+        bool ok;
+        const float* p = src.row(lo + ((4 * q + wave) % (ROWS / 16)) * 16 + rl, ok);
+        v[q] = load4(p, k0 + ((4 * q + wave) / (ROWS / 16)) * 16 + 4 * cl, ok);
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dst[(c + e) * RS + r] = v[e];
+    for (int q = 0; q < NV; ++q) {
+        const int r = ((4 * q + wave) % (ROWS / 16)) * 16 + rl;
+        const int c = ((4 * q + wave) / (ROWS / 16)) * 16 + 4 * cl;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[(c + e) * RS + r] = v[q][e];
     }
 }
 
 // dst[r][i] = row lo + r, RS floats per row.
 template <int ROWS, int HD, int RS>
 __device__ inline void stage_by_row(float* dst, const TokRows& src, int lo) {
-    constexpr int C4 = HD / 4;
+    constexpr int C4 = HD / 4, NV = ROWS * C4 / 256;
+    const int r = threadIdx.x / C4, c = 4 * (threadIdx.x % C4);
+    f32x4 v[NV];
 #pragma unroll
-    for (int e0 = 0; e0 < ROWS * C4; e0 += 256) {
-        const int e = e0 + threadIdx.x, r = e / C4, c = 4 * (e % C4);
-        *reinterpret_cast<f32x4*>(dst + r * RS + c) = load4(src.row(lo + r), c);
+    for (int q = 0; q < NV; ++q) {
+        bool ok;
+        const float* p = src.row(lo + r + q * (256 / C4), ok);
+        v[q] = load4(p, c, ok);
     }
+#pragma unroll
+    for (int q = 0; q < NV; ++q) *reinterpret_cast<f32x4*>(dst + (r + q * (256 / C4)) * RS + c) = v[q];
 }
 
 // out[r] = sum_w A(r, w) Z[w], A(r, w) = sum_i X[r][i] Y[w][i] G[d][i].  FWD: rows are steps t
@@ -634,19 +656,22 @@ fac_tok_pair_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
     for (int i = 0; i < 4; ++i) {
         const int r = rb * kTokB + 16 * wave + 4 * g + i;
         if (r >= L) continue;
-        const bool ok = FWD || ek.row(r);
+        bool ok = true;
+        if (!FWD) ek.row(r, ok);
 #pragma unroll
         for (int j = 0; j < HD / 16; ++j) out[slice + (int64_t)r * D + 16 * j + c16] = ok ? acc[j][i] : 0.f;
     }
 }
 
-// The A or B operands of a product over the dimensions of row p: lane group g holds dimensions
+// The A or B operands of a product over the dimensions of row r: lane group g holds dimensions
 // 16 q + 4 g + e of step 4 q + e (the sum over k takes them in any order).
 template <int HD>
-__device__ inline void dim_operand(const float* p, int g, float (&v)[HD / 4]) {
+__device__ inline void dim_operand(const TokRows& src, int r, int g, float (&v)[HD / 4]) {
+    bool ok;
+    const float* p = src.row(r, ok);
 #pragma unroll
     for (int q = 0; q < HD / 16; ++q) {
-        const f32x4 t = load4(p, 16 * q + 4 * g);
+        const f32x4 t = load4(p, 16 * q + 4 * g, ok);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[4 * q + e] = t[e];
     }
@@ -713,12 +738,12 @@ fac_tok_gate_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
 #pragma unroll
     for (int a = 0; a < TT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
     float xv[HD / 4];
-    dim_operand<HD>(xr.row(rb * kTokB + 16 * wave + c16), g, xv);
+    dim_operand<HD>(xr, rb * kTokB + 16 * wave + c16, g, xv);
     const int w_lo = ROWT ? 0 : rb, w_hi = ROWT ? rb : nb - 1;
     for (int wb = w_lo; wb <= w_hi; ++wb) {
         float zv[4][HD / 4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dim_operand<HD>(zr.row(wb * kTokB + 16 * j + c16), g, zv[j]);
+        for (int j = 0; j < 4; ++j) dim_operand<HD>(zr, wb * kTokB + 16 * j + c16, g, zv[j]);
         __syncthreads();
         stage_by_row<kTokB, HD, HD>(Ys, yr, wb * kTokB);
         stage_by_row<2 * kTokB, HD, HD>(Gs, gt, (ROWT ? rb - wb : wb - rb) * kTokB - (kTokB - 1));
@@ -746,7 +771,8 @@ fac_tok_gate_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
     for (int a = 0; a < TT; ++a) {
         const int r = rb * kTokB + 16 * wave + rg + a;
         if (r >= L) continue;
-        const bool ok = ROWT || ev.row(r);
+        bool ok = true;
+        if (!ROWT) ev.row(r, ok);
         *reinterpret_cast<f32x4u*>(out + slice + (int64_t)r * D + ig) = ok ? acc[a] : f32x4{0.f, 0.f, 0.f, 0.f};
     }
 }
@@ -777,9 +803,9 @@ fac_tok_dist_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
     for (int tb = db; tb < nb; ++tb) {
         const int slo = (tb - db) * kTokB - (kTokB - 1);
         float xv[HD / 4], zv[5][HD / 4];
-        dim_operand<HD>(go.row(tb * kTokB + 16 * wave + c16), g, xv);
+        dim_operand<HD>(go, tb * kTokB + 16 * wave + c16, g, xv);
 #pragma unroll
-        for (int j = 0; j < 5; ++j) dim_operand<HD>(ev.row(slo + 16 * (wave + j) + c16), g, zv[j]);
+        for (int j = 0; j < 5; ++j) dim_operand<HD>(ev, slo + 16 * (wave + j) + c16, g, zv[j]);
         __syncthreads();
         stage_by_row<kTokB, HD, HD>(Qs, qr, tb * kTokB);
         stage_by_row<2 * kTokB, HD, HD>(Es, ek, slo);
