@@ -228,6 +228,42 @@ def test_gpu_reference_scenarios():
     assert total == sum(len(d) - 1 for d in docs)
 
 
+@pytest.mark.parametrize("V", [1, 63, 64, 65, 4097, 131072, 131073, 300001])
+def test_gpu_slot_lists_by_vocabulary(V):
+    """mb_slot_lists at the edges of its words (64 ids) and tiles (131 072 ids): chunk tokens in id
+    order, then the history-only tokens in id order; the last row is not a valid chunk."""
+    from mathbrain import _lib
+    rng = np.random.default_rng(V)
+    T = 3000
+    tokens = rng.integers(0, V, T).astype(np.int32)
+    tokens[rng.integers(0, T, 40)] = V - 1
+    nxt = np.full(T, T, np.int32)
+    seen = {}
+    for p in range(T - 1, -1, -1):
+        nxt[p] = seen.get(int(tokens[p]), T)
+        seen[int(tokens[p])] = p
+    rows = [(0, 0, 500), (0, 2500, 3000), (100, 101, 102), (50, 40, 60)]
+    B = len(rows)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    tk, nx = dev(tokens), dev(nxt)
+    ds, st, en = (dev(np.array(c, np.int64)) for c in zip(*rows))
+    last = torch.empty(B, V, dtype=torch.int32, device="cuda")
+    slot_of = torch.empty(B, V, dtype=torch.int32, device="cuda")
+    slot_tok = torch.full((B, V), -7, dtype=torch.int64, device="cuda")
+    counts = torch.empty(B, 2, dtype=torch.int32, device="cuda")
+    _lib.call("mb_slot_lists", _lib.ptr(tk), _lib.ptr(nx), T, V, _lib.ptr(ds), _lib.ptr(st), _lib.ptr(en), B,
+              _lib.ptr(last), _lib.ptr(slot_of), _lib.ptr(slot_tok), _lib.ptr(counts), _lib.stream(tk.device))
+    for b, (d, s, e) in enumerate(rows):
+        own = np.unique(tokens[s:e]) if s >= d else np.empty(0, np.int64)
+        before = np.setdiff1d(np.unique(tokens[d:s]), own) if s >= d else own
+        want = np.concatenate([own, before])
+        assert counts[b].tolist() == [len(own), len(want)]
+        assert slot_tok[b, :len(want)].tolist() == want.tolist()
+        inverse = np.full(V, -1)
+        inverse[want.astype(np.int64)] = np.arange(len(want))
+        assert np.array_equal(slot_of[b].cpu().numpy(), inverse)
+
+
 def test_gpu_slot_loader_matches_get_batch():
     from mathbrain.data import SlotBatchLoader, TokenBudgetSampler, dynamic_collate_fn
     from mathbrain.synthetic import zipf_corpus
