@@ -107,7 +107,8 @@ def _build_unique_index(x, device, width=None):
         ids, _ = unique_rows(x, K_max)
         return ids.to(x.dtype), K_max
     ids, counts = unique_rows(x, max(L, 16))
-    lo, hi = (int(v) for v in counts.aminmax()) if counts.numel() else (0, 0)
+    found = counts.tolist()  # one read-back for both ends
+    lo, hi = (min(found), max(found)) if found else (0, 0)
     if lo < 0:
         raise _lib.HipKernelError("_build_unique_index: a row of more than 8192 ids spans 2^32 or more "
                                   "(rows that long are sorted as 32-bit offsets)")
