@@ -497,8 +497,8 @@ __device__ inline bool tok_ok(int64_t v, int64_t V) { return v >= 0 && v < V; }
 // dimension (A in the forward and for dE_v, dQ, dE_k and dG: 10 in all), and next to it the LDS
 // reads, 3 or 4 of 16 bytes per 32 operations.  Lanes as steps with whole rows in registers
 // instead read G from LDS for every pair and dimension, and the other rows once per wave.
-// B56 T512 H8 head_dim 64, forward + backward: 9.4 -> 3.9 ms (o 0.78, dE_v 0.67, dQ 0.78,
-// dE_k 0.68, dG 1.00); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.61 ms.
+// B56 T512 H8 head_dim 64, forward + backward: 9.4 -> 3.5 ms (o 0.73, dE_v 0.64, dQ 0.63,
+// dE_k 0.66, dG 0.84); B5 T253 H4 head_dim 32, the whole call: 1.76 -> 1.60 ms.
 
 constexpr int kTokB = 64;  // steps per block
 
@@ -511,16 +511,19 @@ struct TokRows {
     const int64_t* ids;
     int64_t V, D;
     int L;
-    __device__ inline const float* row(int r, bool& ok) const {
+    __device__ inline int64_t id(int r) const {
+        const int64_t v = min(max(r, 0), L - 1);
+        return ids ? ids[v] : v;
+    }
+    __device__ inline const float* at(int64_t v, int r, bool& ok) const {  // v = id(r)
         ok = r >= 0 && r < L;
-        int64_t v = min(max(r, 0), L - 1);
         if (ids) {
-            v = ids[v];
             ok = ok && tok_ok(v, V);
             v = tok_ok(v, V) ? v : 0;
         }
         return p + v * D;
     }
+    __device__ inline const float* row(int r, bool& ok) const { return at(id(r), r, ok); }
 };
 
 __device__ inline f32x4 load4(const float* p, int c, bool ok) {
@@ -531,43 +534,61 @@ __device__ inline f32x4 load4(const float* p, int c, bool ok) {
     return o;
 }
 
-// dst[k][r] = rows lo + r, dimensions k0 + k, for ROWS x KC; RS floats per dimension.  Four lanes
-// on 64 bytes of a row and 16 rows per wave: the transposed writes use every bank twice.
+// A thread's part of dimensions k0 .. k0 + KC - 1 of rows lo .. lo + ROWS - 1, stored to dst[k][r] (RS
+// floats per dimension).  Four lanes on 64 bytes of a row and 16 rows per wave: the transposed
+// writes use every bank twice.
 template <int ROWS, int KC, int RS>
-__device__ inline void stage_by_dim(float* dst, const TokRows& src, int lo, int k0) {
-    constexpr int NV = (ROWS / 16) * (KC / 16) / 4;
-    const int cl = threadIdx.x & 3, rl = (threadIdx.x >> 2) & 15, wave = threadIdx.x >> 6;
+struct DimPiece {
+    static constexpr int RT = ROWS / 16, NV = RT * (KC / 16) / 4;
     f32x4 v[NV];
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        bool ok;
-        const float* p = src.row(lo + ((4 * q + wave) % (ROWS / 16)) * 16 + rl, ok);
-        v[q] = load4(p, k0 + ((4 * q + wave) / (ROWS / 16)) * 16 + 4 * cl, ok);
+    __device__ static inline int row(int q) {
+        return ((4 * q + (threadIdx.x >> 6)) % RT) * 16 + ((threadIdx.x >> 2) & 15);
     }
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        const int r = ((4 * q + wave) % (ROWS / 16)) * 16 + rl;
-        const int c = ((4 * q + wave) / (ROWS / 16)) * 16 + 4 * cl;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dst[(c + e) * RS + r] = v[q][e];
+    __device__ static inline int dim(int q) {
+        return ((4 * q + (threadIdx.x >> 6)) / RT) * 16 + 4 * (threadIdx.x & 3);
     }
-}
+    __device__ inline void load(const TokRows& src, int lo, int k0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            bool ok;
+            const float* p = src.row(lo + row(q), ok);
+            v[q] = load4(p, k0 + dim(q), ok);
+        }
+    }
+    __device__ inline void store(float* dst) const {
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dst[(dim(q) + e) * RS + row(q)] = v[q][e];
+    }
+};
 
-// dst[r][i] = row lo + r, RS floats per row.
+// A thread's part of rows lo .. lo + ROWS - 1: their ids, the loads, and the store to dst[r][i] (RS
+// floats per row).  The three are apart so that a tile's ids and rows are on their way while the
+// tile before it is computed (3.9 -> 3.5 ms).
 template <int ROWS, int HD, int RS>
-__device__ inline void stage_by_row(float* dst, const TokRows& src, int lo) {
-    constexpr int C4 = HD / 4, NV = ROWS * C4 / 256;
-    const int r = threadIdx.x / C4, c = 4 * (threadIdx.x % C4);
+struct RowPiece {
+    static constexpr int C4 = HD / 4, NV = ROWS * C4 / 256, STEP = 256 / C4;
+    int64_t id[NV];
     f32x4 v[NV];
+    __device__ inline void ids(const TokRows& src, int lo) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        bool ok;
-        const float* p = src.row(lo + r + q * (256 / C4), ok);
-        v[q] = load4(p, c, ok);
+        for (int q = 0; q < NV; ++q) id[q] = src.id(lo + threadIdx.x / C4 + q * STEP);
     }
+    __device__ inline void load(const TokRows& src, int lo) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) *reinterpret_cast<f32x4*>(dst + (r + q * (256 / C4)) * RS + c) = v[q];
-}
+        for (int q = 0; q < NV; ++q) {
+            bool ok;
+            const float* p = src.at(id[q], lo + threadIdx.x / C4 + q * STEP, ok);
+            v[q] = load4(p, 4 * (threadIdx.x % C4), ok);
+        }
+    }
+    __device__ inline void store(float* dst) const {
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+            *reinterpret_cast<f32x4*>(dst + (threadIdx.x / C4 + q * STEP) * RS + 4 * (threadIdx.x % C4)) = v[q];
+    }
+};
 
 // out[r] = sum_w A(r, w) Z[w], A(r, w) = sum_i X[r][i] Y[w][i] G[d][i].  FWD: rows are steps t
 // and the walked ones s < t (O); otherwise rows are steps s and the walked ones t > s (dE_v).
@@ -596,11 +617,26 @@ fac_tok_pair_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
     f32x4 acc[HD / 16];
 #pragma unroll
     for (int j = 0; j < HD / 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    stage_by_dim<kTokB, HD, RS>(Xs, xr, rb * kTokB, 0);
+    {
+        DimPiece<kTokB, HD, RS> px;
+        px.load(xr, rb * kTokB, 0);
+        px.store(Xs);
+    }
     const float* gbase = Gs + (FWD ? 4 * (ty - tx) : 4 * (tx - ty)) + 60;
     const int w_lo = FWD ? 0 : rb, w_hi = FWD ? rb : nb - 1;
+    DimPiece<kTokB, KC, RS> py;
+    DimPiece<2 * kTokB, KC, GS> pg;
+    RowPiece<kTokB, HD, ZS> pz;
+    auto load = [&](int wb, int kc) {
+        py.load(yr, wb * kTokB, kc);
+        pg.load(gt, (FWD ? rb - wb : wb - rb) * kTokB - (kTokB - 1), kc);
+        if (kc == 0) {
+            pz.ids(z, wb * kTokB);
+            pz.load(z, wb * kTokB);
+        }
+    };
+    load(w_lo, 0);
     for (int wb = w_lo; wb <= w_hi; ++wb) {
-        const int dlo = (FWD ? rb - wb : wb - rb) * kTokB - (kTokB - 1);
         float a[4][4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -609,9 +645,11 @@ fac_tok_pair_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
 #pragma unroll
         for (int kc = 0; kc < HD; kc += KC) {
             __syncthreads();
-            stage_by_dim<kTokB, KC, RS>(Ys, yr, wb * kTokB, kc);
-            stage_by_dim<2 * kTokB, KC, GS>(Gs, gt, dlo, kc);
-            if (kc == 0) stage_by_row<kTokB, HD, ZS>(Zs, z, wb * kTokB);
+            py.store(Ys);
+            pg.store(Gs);
+            if (kc == 0) pz.store(Zs);
+            if (kc + KC < HD) load(wb, kc + KC);
+            else load(min(wb + 1, w_hi), 0);
             __syncthreads();
 #pragma unroll 4
             for (int k = 0; k < KC; ++k) {
@@ -666,9 +704,9 @@ fac_tok_pair_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
 // The A or B operands of a product over the dimensions of row r: lane group g holds dimensions
 // 16 q + 4 g + e of step 4 q + e (the sum over k takes them in any order).
 template <int HD>
-__device__ inline void dim_operand(const TokRows& src, int r, int g, float (&v)[HD / 4]) {
+__device__ inline void dim_operand(const TokRows& src, int64_t id, int r, int g, float (&v)[HD / 4]) {
     bool ok;
-    const float* p = src.row(r, ok);
+    const float* p = src.at(id, r, ok);
 #pragma unroll
     for (int q = 0; q < HD / 16; ++q) {
         const f32x4 t = load4(p, 16 * q + 4 * g, ok);
@@ -738,15 +776,35 @@ fac_tok_gate_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
 #pragma unroll
     for (int a = 0; a < TT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
     float xv[HD / 4];
-    dim_operand<HD>(xr, rb * kTokB + 16 * wave + c16, g, xv);
+    {
+        const int r = rb * kTokB + 16 * wave + c16;
+        dim_operand<HD>(xr, xr.id(r), r, g, xv);
+    }
     const int w_lo = ROWT ? 0 : rb, w_hi = ROWT ? rb : nb - 1;
-    for (int wb = w_lo; wb <= w_hi; ++wb) {
-        float zv[4][HD / 4];
+    RowPiece<kTokB, HD, HD> py;
+    RowPiece<2 * kTokB, HD, HD> pg;
+    int64_t zid[4];
+    float zv[4][HD / 4];
+    auto ids = [&](int wb) {
+        py.ids(yr, wb * kTokB);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dim_operand<HD>(zr, wb * kTokB + 16 * j + c16, g, zv[j]);
+        for (int j = 0; j < 4; ++j) zid[j] = zr.id(wb * kTokB + 16 * j + c16);
+    };
+    auto load = [&](int wb) {
+        const int dlo = (ROWT ? rb - wb : wb - rb) * kTokB - (kTokB - 1);
+        pg.ids(gt, dlo);
+        pg.load(gt, dlo);
+        py.load(yr, wb * kTokB);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dim_operand<HD>(zr, zid[j], wb * kTokB + 16 * j + c16, g, zv[j]);
+    };
+    ids(w_lo);
+    load(w_lo);
+    for (int wb = w_lo; wb <= w_hi; ++wb) {
+        ids(min(wb + 1, w_hi));
         __syncthreads();
-        stage_by_row<kTokB, HD, HD>(Ys, yr, wb * kTokB);
-        stage_by_row<2 * kTokB, HD, HD>(Gs, gt, (ROWT ? rb - wb : wb - rb) * kTokB - (kTokB - 1));
+        py.store(Ys);
+        pg.store(Gs);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             f32x4 d = {0.f, 0.f, 0.f, 0.f};
@@ -761,6 +819,7 @@ fac_tok_gate_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
             }
             *reinterpret_cast<f32x4*>(da + (16 * j + c16) * WS + 4 * g) = d;
         }
+        load(min(wb + 1, w_hi));
         __syncthreads();
         // distance of row r and walked step w: row r - w + 63 of the staged ones (ROWT), w - r + 63
         const int r0 = 16 * wave + rg;
@@ -800,15 +859,33 @@ fac_tok_dist_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
     f32x4 acc[TT];
 #pragma unroll
     for (int a = 0; a < TT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    RowPiece<kTokB, HD, HD> pq;
+    RowPiece<2 * kTokB, HD, HD> pe;
+    int64_t zid[5];
+    auto ids = [&](int tb) {
+        const int slo = (tb - db) * kTokB - (kTokB - 1);
+        pe.ids(ek, slo);
+#pragma unroll
+        for (int j = 0; j < 5; ++j) zid[j] = ev.id(slo + 16 * (wave + j) + c16);
+    };
+    auto load = [&](int tb) {
+        pq.ids(qr, tb * kTokB);
+        pq.load(qr, tb * kTokB);
+        pe.load(ek, (tb - db) * kTokB - (kTokB - 1));
+    };
+    ids(db);
+    load(db);
     for (int tb = db; tb < nb; ++tb) {
         const int slo = (tb - db) * kTokB - (kTokB - 1);
+        const int next = min(tb + 1, nb - 1);
         float xv[HD / 4], zv[5][HD / 4];
-        dim_operand<HD>(go, tb * kTokB + 16 * wave + c16, g, xv);
+        dim_operand<HD>(go, go.id(tb * kTokB + 16 * wave + c16), tb * kTokB + 16 * wave + c16, g, xv);
 #pragma unroll
-        for (int j = 0; j < 5; ++j) dim_operand<HD>(ev, slo + 16 * (wave + j) + c16, g, zv[j]);
+        for (int j = 0; j < 5; ++j) dim_operand<HD>(ev, zid[j], slo + 16 * (wave + j) + c16, g, zv[j]);
         __syncthreads();
-        stage_by_row<kTokB, HD, HD>(Qs, qr, tb * kTokB);
-        stage_by_row<2 * kTokB, HD, HD>(Es, ek, slo);
+        pq.store(Qs);
+        pe.store(Es);
+        ids(next);
 #pragma unroll
         for (int j = 0; j < 5; ++j) {
             f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -821,6 +898,7 @@ fac_tok_dist_kernel(const float* __restrict__ Q, const float* __restrict__ dO, c
                 if (d >= 0 && d < kTokB) dAs[t * WS + d] = slo + si >= 0 && db + d > 0 && tb * kTokB + t < L ? v[i] : 0.f;
             }
         }
+        load(next);
         __syncthreads();
         const int d0 = 16 * wave + rg;
         gate_rows<HD, 1, WS>(dAs + d0, Qs, Es, kTokB - 1 - d0, ig, acc);
