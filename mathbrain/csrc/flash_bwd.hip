@@ -623,8 +623,13 @@ static size_t bwd_lds_bytes() {
            (SUB ? (size_t)2 * kBwdHeads * 2 * 32 * 4 : 0);
 }
 
+// Bytes of one workgroup's dW_pe sums: the columns of four waves' dims (head_dim 128 runs as
+// 64-dim sub-heads) x the instantiation's rates.
+constexpr int64_t bwd_dw_bytes(int hd, int tiles) { return (int64_t)kBwdHeads * (hd < 64 ? hd : 64) * 32 * tiles * 4; }
+
+// part_bytes: size of a.dWpart
 template <int HD, int NS, int SB, bool PG = false, bool PW = false, bool SUB = false>
-static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, hipStream_t st) {
+static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, int64_t part_bytes, hipStream_t st) {
     FlashArgsV a = a0;
     // heads per group: the largest divisor of H that is at most four (with SUB two heads,
     // whose four sub-heads take the four wave pairs)
@@ -643,6 +648,7 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, hipStream_t 
     constexpr int NTW = NT < 256 / HD ? NT : 256 / HD;
     constexpr bool XH = NT > NTW;
     static_assert(NT == NTW || NT == 2 * NTW, "at most two half-waves per head");
+    static_assert(bwd_dw_bytes(HD, NS) == (int64_t)kBwdHeads * (HD / 16) * NT * 64 * 16, "one f32x4 per lane and tile");
     const size_t lds = std::max(bwd_lds_bytes<HD, NS, SB, XH, PG, PW, SUB>(),
                                 XH ? (size_t)0 : (size_t)kBwdHeads * (HD / 16) * NTW * 64 * 16);  // dW_pe's halves
     if (lds > 160 * 1024)
@@ -657,7 +663,7 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, hipStream_t 
     const int64_t G = (int64_t)a.B * ntb * a.head_groups;
     a.ksplit = slot_parts(G, conc, (a.K + SB - 1) / SB);
     const int64_t wgs = G * a.ksplit;
-    if (wgs > conc) a.dWpart = nullptr;
+    if (wgs > conc || part_bytes < wgs * bwd_dw_bytes(HD, NS)) a.dWpart = nullptr;
     if (a.ksplit > 1) {
         zero.p[3] = a.dQ;
         zero.n[3] = (int64_t)a.B * a.H * a.L * a.hd;
@@ -706,8 +712,7 @@ using namespace mb;
 
 extern "C" int64_t mb_flash_ema_bwd_workspace(int hd, int N) {
     if (hd < 1 || N < 1) return 0;
-    // a workgroup's dW_pe tile: its head group's columns x the rates rounded up to whole tiles
-    return (int64_t)device_cus() * kBwdHeads * std::min(hd, 64) * ((N + 31) / 32 * 32) * 4;
+    return device_cus() * bwd_dw_bytes(hd, rate_tiles(N));
 }
 
 extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
@@ -732,7 +737,8 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     flash_use_lists(a, slot_lists);
     MB_REQUIRE(workspace_bytes >= 0, "mb_flash_ema_bwd: negative workspace size %lld", (long long)workspace_bytes);
     MB_REQUIRE(((uintptr_t)workspace & 15) == 0, "mb_flash_ema_bwd: workspace must be 16-byte aligned");
-    if (workspace && workspace_bytes >= mb_flash_ema_bwd_workspace(hd, N)) a.dWpart = static_cast<float*>(workspace);
+    a.dWpart = static_cast<float*>(workspace);
+    const int64_t part_bytes = workspace ? workspace_bytes : 0;
     const bool vr = (flags & MB_FLASH_VOCAB_ROWS) != 0;
     a.e_rows = vr ? V_total : 0;
     int rc = flash_validate("mb_flash_ema_bwd", a, hd);
@@ -752,7 +758,7 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     MB_REQUIRE(Q && dO && x && rhos && unique && O && LSE && W_pe && dQ,
                "mb_flash_ema_bwd: null pointer");
     MB_REQUIRE(K == 0 || (E_k && E_v && C_bounds), "mb_flash_ema_bwd: null slot pointer");
-    const int NS = (N + 31) / 32;
+    const int NS = rate_tiles(N);
     const int gm = flash_gate_mode("mb_flash_ema_bwd", flags, N, hd);
     if (gm < 0) return gm;
     if (gm == 2) {
@@ -761,26 +767,26 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
         // a batch's barrier, loads and stores are shared by its slots, and a slot of 32 dims is
         // too short to cover them (B3 T201 H6 N33: backward 449 us with one slot per batch, 356 us
         // with two).
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, zero, st) : launch_bwd<64, 2, 1, true, true>(a, vr, zero, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, zero, st) : launch_bwd<32, 2, 2, true, true>(a, vr, zero, st);
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, zero, part_bytes, st) : launch_bwd<64, 2, 1, true, true>(a, vr, zero, part_bytes, st);
+        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, zero, part_bytes, st) : launch_bwd<32, 2, 2, true, true>(a, vr, zero, part_bytes, st);
     }
     if (gm == 1) {  // the gate's lo tile and W_lo beside the hi ones
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, zero, st) : launch_bwd<64, 2, 2, true>(a, vr, zero, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, zero, st) : launch_bwd<32, 2, 2, true>(a, vr, zero, st);
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, zero, part_bytes, st) : launch_bwd<64, 2, 2, true>(a, vr, zero, part_bytes, st);
+        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, zero, part_bytes, st) : launch_bwd<32, 2, 2, true>(a, vr, zero, part_bytes, st);
     }
     if (hd == 128) {  // two 64-dim sub-heads per head
-        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, zero, st);
-        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, zero, st);
-        return launch_bwd<64, 4, 1, false, false, true>(a, vr, zero, st);
+        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, zero, part_bytes, st);
+        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, zero, part_bytes, st);
+        return launch_bwd<64, 4, 1, false, false, true>(a, vr, zero, part_bytes, st);
     }
     if (hd == 64) {
-        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, zero, st);
-        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, zero, st);
-        return launch_bwd<64, 4, 1>(a, vr, zero, st);
+        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, zero, part_bytes, st);
+        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, zero, part_bytes, st);
+        return launch_bwd<64, 4, 1>(a, vr, zero, part_bytes, st);
     }
-    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, zero, st);
-    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, zero, st);
-    return launch_bwd<32, 4, 2>(a, vr, zero, st);
+    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, zero, part_bytes, st);
+    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, zero, part_bytes, st);
+    return launch_bwd<32, 4, 2>(a, vr, zero, part_bytes, st);
 }
 
 extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,

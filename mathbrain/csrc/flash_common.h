@@ -287,6 +287,11 @@ struct Stage {
     }
 };
 
+// 32-rate tiles of the instantiation that takes N rates: the kernels are built for 1, 2 and 4, so
+// N = 65 .. 96 runs with four, the last of them zeros.  What a kernel writes per rate is sized by
+// this, not by N.
+static inline int rate_tiles(int N) { return N <= 32 ? 1 : N <= 64 ? 2 : 4; }
+
 // Gate arithmetic of a flash-EMA call, the same in the forward and the backward:
 // 2 = MB_FLASH_FP32 (split gate and split dW_pe product), 1 = the default's split gate with
 // bf16 dW_pe operands, 0 = single fp16 gate products (MB_FLASH_FAST_GATE, and the default

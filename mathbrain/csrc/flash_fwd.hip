@@ -32,7 +32,7 @@ using namespace mb;
 // plans the slot split (see launch_fwd).
 static int fwd_dispatch(const FlashArgsV& a, int hd, int N, int flags, bool vr, hipStream_t st, float* part,
                         int64_t ws_bytes, int64_t* ws_need) {
-    const int NS = (N + 31) / 32;
+    const int NS = rate_tiles(N);
     const int gm = flash_gate_mode("mb_flash_ema_fwd", flags, N, hd);
     if (gm < 0) return gm;
     if (gm > 0) {

@@ -61,7 +61,7 @@ extern "C" int mb_flash_ema_fwd_gq(const float* x_q, int64_t xq_sb, int64_t xq_s
     MB_REQUIRE(x && rhos && unique && O && LSE && W_pe, "mb_flash_ema_fwd_gq: null pointer");
     MB_REQUIRE(K == 0 || (E_k && E_v && C_bounds), "mb_flash_ema_fwd_gq: null slot pointer");
     hipStream_t st = (hipStream_t)stream;
-    const int NS = (N + 31) / 32;
+    const int NS = rate_tiles(N);
     const int gm = flash_gate_mode("mb_flash_ema_fwd_gq", flags, N, hd);
     if (gm < 0) return gm;
     if (gm > 0) {

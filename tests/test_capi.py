@@ -98,6 +98,18 @@ def test_data_and_factored_argument_errors_need_no_gpu(lib):
     assert rc == _lib.MB_ERR_UNSUPPORTED and b"head_dim=16" in L.mb_last_error()
 
 
+@pytest.mark.parametrize("hd", [32, 64, 128])
+def test_backward_workspace_holds_every_workgroup(lib, hd):
+    """mb_flash_ema_bwd_workspace: room for the dW_pe sums of a workgroup per compute unit (256),
+    whose kernel runs with 1, 2 or 4 tiles of 32 rates: four from N = 65 on, also where three
+    would hold N."""
+    from mathbrain import _lib
+    for N in range(1, 129):
+        rates = 32 if N <= 32 else 64 if N <= 64 else 128
+        a_workgroup = 4 * 4 * min(hd, 64) * rates      # fp32, four waves of at most 64 dims
+        assert _lib.lib().mb_flash_ema_bwd_workspace(hd, N) >= 256 * a_workgroup, N
+
+
 def test_factored_and_data_cpu_tensors_are_rejected():
     import torch
     from mathbrain.factored_ema import factored_ema_forward

@@ -262,6 +262,37 @@ def test_bwd_rates(N, stored_scores, precision):
                    precision=precision)
 
 
+@pytest.mark.parametrize("B, L, H, hd, slots, N", [
+    (2, 128, 4, 32, 128, 80), (1, 512, 8, 64, 250, 80), (1, 512, 4, 128, 250, 96), (2, 128, 4, 32, 128, 65)])
+def test_bwd_rates_between_two_tile_counts(B, L, H, hd, slots, N):
+    """65 to 96 rates run with four rate tiles.  Grids that the slot parts fill to about a workgroup
+    per compute unit, each of which leaves its dW_pe sums in the workspace: nothing past the
+    workspace is written, and the gradients are the oracle's, with the workspace and without."""
+    from mathbrain import _lib
+    from mathbrain.triton_flash_ema import _flash_flags, flash_ema_forward
+    c = make_case(B, L, slots, H, hd, N, warmup=3000, seed=N, uniform=True, qs=0.5, es=0.3, ws=0.2)
+    assert c["K"] == slots
+    check_forward(c)
+    check_backward(c)
+    dO = torch.randn(c["Q"].shape, generator=torch.Generator().manual_seed(77))
+    want = oracle_backward(c, dO, gate_round=case_rounding(c))
+    cu = lambda k: c[k].float().contiguous().cuda()
+    Q, Ek, Ev, W, rh, Cb = (cu(k) for k in ("Q", "E_k", "E_v", "W", "rhos", "Cb"))
+    x, u, dOg = c["x"].cuda(), c["unique"].cuda(), dO.cuda()
+    O, LSE, *_, S2 = flash_ema_forward(Q, x, Ek, Ev, W, rh, c["V"], u, c["K"], Cb, Br=c["Br"], return_scores=True)
+    size, past = _lib.lib().mb_flash_ema_bwd_workspace(hd, N), 1 << 24
+    p = _lib.ptr
+    for ws_bytes in (size, 0):
+        buf = torch.full((size + past,), 0x5A, dtype=torch.uint8, device="cuda")
+        g = [torch.full(t.shape, float("nan"), device="cuda") for t in (Q, Ek, Ev, W)]
+        _lib.call("mb_flash_ema_bwd_lists", p(Q), *Q.stride(), p(dOg), p(x), x.stride(0), x.stride(1), p(Ek), p(Ev),
+                  p(W), p(rh), p(u), p(Cb), p(O), p(LSE), B, H, L, hd, c["K"], N, Cb.shape[3], Cb.shape[1], c["Br"],
+                  c["V"], _flash_flags(True, True), p(S2), *(p(t) for t in g), None, p(buf) if ws_bytes else None,
+                  ws_bytes, _lib.stream(Q.device))
+        assert bool((buf[size:] == 0x5A).all())
+        assert max(norm_err(a, b) for a, b in zip(g, want)) < TOL_KERNEL_ROUNDING
+
+
 def test_bwd_cfg2_slice_exact():
     check_backward(make_case(1, 256, 50257, 8, 64, 64, warmup=4096, seed=12, **CFG), exact=True)
 
