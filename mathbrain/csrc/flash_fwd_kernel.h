@@ -430,17 +430,33 @@ flash_fwd_merge_kernel(const float* __restrict__ part, int ks, int64_t rows, flo
     if (c == 0) LSE[r] = any ? (M + __log2f(l)) * kLn2 : -INFINITY;
 }
 
-// Slot parts of the forward: slot_parts for a grid below two rounds of `conc` workgroups.
-// Beyond that the workgroups of equally long lists end their rounds together, and a split
-// must save at least 3 % of the rounds: 896 at B56 T512 take 4 rounds of 256 where 3.5 would
-// do (two parts: 10.22 -> 9.12 ms with single products), and keep four batches per part.
+// Slot parts of the forward.  A grid below two rounds of `conc` workgroups takes those of
+// slot_parts, which even out lists of different lengths, or up to four more where that shortens
+// equally long ones by at least 7.5 %: rounds x (batches of a part + kPartPrice, what a part
+// repeats).  448 workgroups at B28 T512 H8 N64 take 6 rounds of 256 in slot_parts' three parts
+// (2.0 of a whole walk), 7 in four (1.75): 6.45 -> 5.73 ms; 288 with 150 slots take two rounds whole, 5 in
+// four parts: 654 -> 527 us.  Batches of documents pay up to 7 % for it (B11 0.94 -> 1.00 ms); fewer
+// parts than slot_parts' would cost them more (four for seven: 1.32 ms).
+// From two rounds on the workgroups of equally long lists end their rounds together, and a split
+// must save at least 3 % of them: 896 at B56 T512 take 4 where 3.5 would do (two parts: 10.22 ->
+// 9.12 ms with single products).  Every part keeps four batches.
+constexpr double kPartPrice = 4.0;
 static int fwd_parts(int64_t G, int64_t conc, int nbatch) {
-    if (G < 2 * conc) return slot_parts(G, conc, nbatch);
+    if (G <= 0 || conc <= 0) return 1;
+    auto rounds = [&](int ks) { return (double)((G * ks + conc - 1) / conc); };
+    if (G < 2 * conc) {
+        auto cost = [&](int ks) { return rounds(ks) * ((double)nbatch / ks + kPartPrice); };
+        const int even = slot_parts(G, conc, nbatch);
+        int best = even;
+        for (int ks = even + 1; ks <= even + 4 && nbatch >= 4 * ks; ++ks)
+            if (cost(ks) < cost(best)) best = ks;
+        return cost(best) < 0.925 * cost(even) ? best : even;
+    }
     int best = 1;
-    double best_cost = (double)((G + conc - 1) / conc);
+    double best_cost = rounds(1);
     for (int ks = 2; ks <= 4; ++ks) {
         if (nbatch < 4 * ks) break;
-        const double cost = (double)((G * ks + conc - 1) / conc) / ks * (1.0 + 0.02 * (ks - 1));
+        const double cost = rounds(ks) / ks * (1.0 + 0.02 * (ks - 1));
         if (cost < 0.97 * best_cost) {
             best = ks;
             best_cost = cost;

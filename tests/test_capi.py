@@ -110,6 +110,22 @@ def test_backward_workspace_holds_every_workgroup(lib, hd):
         assert _lib.lib().mb_flash_ema_bwd_workspace(hd, N) >= 256 * a_workgroup, N
 
 
+@pytest.mark.parametrize("K", [60, 150, 979, 1638])
+def test_forward_parts_fit_the_rounds(lib, K):
+    """The forward's slot parts (read from its workspace: parts x rows x (hd + 2) floats) on grids
+    below two rounds of 256 workgroups.  Where all slot lists are equally long a launch takes
+    rounds x (a part's batches of three slots + 4 for what a part repeats); against the shortest
+    of one to four parts, the parts that even out other lists may cost 4 per 32 batches."""
+    from mathbrain import _lib
+    L, H, hd, N, batches = 512, 8, 64, 64, -(-K // 3)
+    for B in range(1, 32):
+        G = B * L // 32
+        need = _lib.lib().mb_flash_ema_fwd_workspace(B, H, L, hd, K, N, _lib.MB_FLASH_SILU)
+        parts = max(1, need // (B * H * L * (hd + 2) * 4))
+        time = lambda p: -(-G * p // 256) * (batches / p + 4)  # noqa: E731
+        assert time(parts) <= 1.125 * min(time(p) for p in range(1, 5) if p == 1 or batches >= 4 * p), (B, parts)
+
+
 def test_factored_and_data_cpu_tensors_are_rejected():
     import torch
     from mathbrain.factored_ema import factored_ema_forward
