@@ -294,7 +294,10 @@ flash_ema_bwd_kernel(typename FlashArgsOf<VR>::type a) {
         const float* E = E_of(cur);
         const BatchMeta* meta = meta_of(bi);
         for (int j = 0; j < SB; ++j) {
-            const BatchMeta slot = meta[j];
+            // Without the forward's scores the body has no registers left for the slot's row and
+            // index (three spilled: B56 T512 27.05 -> 28.05 ms, in scalar registers 27.51); with
+            // them it has (22.36 ms, 22.55 with the scalar moves).
+            const BatchMeta slot = HAS_S ? meta[j] : uniform_slot(meta[j]);
             if (slot.row < 0) continue;  // padding slot (uniform across the workgroup)
             if (!active) {                // a wave without a head: only the exchange barriers
                 if (SUB) {

@@ -316,6 +316,11 @@ __device__ inline int64_t e_row(const A& a, int b, const BatchMeta& m) {
     return min((int64_t)max(m.row, 0), e_rows_of(a) - 1);
 }
 
+// A batch's slot with its row and index in scalar registers (they are the same in every lane).
+__device__ inline BatchMeta uniform_slot(const BatchMeta& m) {
+    return BatchMeta{0, __builtin_amdgcn_readfirstlane(m.row), __builtin_amdgcn_readfirstlane(m.k)};
+}
+
 // Token id as BatchMeta holds it: ids past 2^31 - 1 clamp (e_row clamps to the table anyway).
 __device__ inline int32_t slot_row(int64_t u) { return (int32_t)min(u, (int64_t)INT32_MAX); }
 
