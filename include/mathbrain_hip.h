@@ -295,12 +295,16 @@ int mb_flash_ema_bwd(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, i
 /*
  * mb_flash_ema_bwd over slot lists (NULL: every slot; see mb_flash_ema_slot_lists).
  *
- *   workspace  NULL, or workspace_bytes >= mb_flash_ema_bwd_workspace(hd, N) bytes of device
- *              memory (16-byte aligned, contents irrelevant, one call's at a time): room for
- *              the workgroups' dW_pe sums where all of them run at once; otherwise, and without
- *              it, they are added with atomics.  Gradients agree either way up to the order of
- *              the sums.
+ *   workspace  NULL, or device memory (16-byte aligned, contents irrelevant, one call's at a
+ *              time): room for the workgroups' dW_pe sums where all of them run at once;
+ *              otherwise, without it or with too little, they are added with atomics.
+ *              Gradients agree either way up to the order of the sums.
+ *
+ * mb_flash_ema_bwd_lists_workspace: the bytes that a call of these shapes and flags uses on the
+ * current device, 0 where it adds with atomics anyway (more workgroups than compute units);
+ * negative for shapes it does not take.  mb_flash_ema_bwd_workspace: enough for any such call.
  */
+int64_t mb_flash_ema_bwd_lists_workspace(int B, int H, int L, int hd, int K, int N, int flags);
 int64_t mb_flash_ema_bwd_workspace(int hd, int N);
 int mb_flash_ema_bwd_lists(const float *Q, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t q_sd,
                            const float *dO, const int64_t *x, int64_t x_sb, int64_t x_sl,

@@ -48,6 +48,7 @@ SIGNATURES = {
                                 _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p, _p,
                                 _p, _p, _p, _i64, _p], _i),
     "mb_flash_ema_bwd_workspace": ([_i, _i], _i64),
+    "mb_flash_ema_bwd_lists_workspace": ([_i, _i, _i, _i, _i, _i, _i], _i64),
     "mb_flash_ema_fwd_gq": ([_p, _i64, _i64, _p, _i64, _i64, _p, _p, _f, _p, _p, _i64, _i64, _p, _p, _p,
                              _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i64, _i, _p, _p, _p], _i),
     "mb_gating_fwd": ([_p, _i64, _p, _i64, _p, _p, _i64, _p, _i, _p, _p, _i64, _i, _i, _f, _p, _p,

@@ -630,9 +630,11 @@ static size_t bwd_lds_bytes() {
 // 64-dim sub-heads) x the instantiation's rates.
 constexpr int64_t bwd_dw_bytes(int hd, int tiles) { return (int64_t)kBwdHeads * (hd < 64 ? hd : 64) * 32 * tiles * 4; }
 
-// part_bytes: size of a.dWpart
+// part_bytes: size of a.dWpart.  With ws_need set it only plans: *ws_need = the bytes that a.dWpart
+// would be used with (0: the launch has more workgroups than compute units).
 template <int HD, int NS, int SB, bool PG = false, bool PW = false, bool SUB = false>
-static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, int64_t part_bytes, hipStream_t st) {
+static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, int64_t part_bytes, hipStream_t st,
+                      int64_t* ws_need) {
     FlashArgsV a = a0;
     // heads per group: the largest divisor of H that is at most four (with SUB two heads,
     // whose four sub-heads take the four wave pairs)
@@ -666,7 +668,12 @@ static int launch_bwd(const FlashArgsV& a0, bool vr, ZeroFill zero, int64_t part
     const int64_t G = (int64_t)a.B * ntb * a.head_groups;
     a.ksplit = slot_parts(G, conc, (a.K + SB - 1) / SB);
     const int64_t wgs = G * a.ksplit;
-    if (wgs > conc || part_bytes < wgs * bwd_dw_bytes(HD, NS)) a.dWpart = nullptr;
+    const int64_t need = wgs > conc ? 0 : wgs * bwd_dw_bytes(HD, NS);
+    if (ws_need) {
+        *ws_need = need;
+        return MB_OK;
+    }
+    if (need == 0 || part_bytes < need) a.dWpart = nullptr;
     if (a.ksplit > 1) {
         zero.p[3] = a.dQ;
         zero.n[3] = (int64_t)a.B * a.H * a.L * a.hd;
@@ -713,9 +720,55 @@ void flash_use_lists(FlashArgs& a, const void* lists);
 
 using namespace mb;
 
+// Picks the kernel instantiation for (hd, N, flags) and launches it, or with ws_need only plans the
+// launch (see launch_bwd).
+static int bwd_dispatch(const FlashArgsV& a, int hd, int N, int flags, bool vr, const ZeroFill& zero,
+                        int64_t part_bytes, hipStream_t st, int64_t* ws_need) {
+    const int NS = rate_tiles(N);
+    const int gm = flash_gate_mode("mb_flash_ema_bwd", flags, N, hd);
+    if (gm < 0) return gm;
+    if (gm == 2) {
+        // hi + lo tiles of both kinds and both W fragment sets in LDS: one slot per batch at
+        // head_dim 64, two (N > 32) or four at head_dim 32, whose W fragments and rows take half:
+        // a batch's barrier, loads and stores are shared by its slots, and a slot of 32 dims is
+        // too short to cover them (B3 T201 H6 N33: backward 449 us with one slot per batch, 356 us
+        // with two).
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, zero, part_bytes, st, ws_need) : launch_bwd<64, 2, 1, true, true>(a, vr, zero, part_bytes, st, ws_need);
+        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, zero, part_bytes, st, ws_need) : launch_bwd<32, 2, 2, true, true>(a, vr, zero, part_bytes, st, ws_need);
+    }
+    if (gm == 1) {  // the gate's lo tile and W_lo beside the hi ones
+        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, zero, part_bytes, st, ws_need) : launch_bwd<64, 2, 2, true>(a, vr, zero, part_bytes, st, ws_need);
+        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, zero, part_bytes, st, ws_need) : launch_bwd<32, 2, 2, true>(a, vr, zero, part_bytes, st, ws_need);
+    }
+    if (hd == 128) {  // two 64-dim sub-heads per head
+        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, zero, part_bytes, st, ws_need);
+        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, zero, part_bytes, st, ws_need);
+        return launch_bwd<64, 4, 1, false, false, true>(a, vr, zero, part_bytes, st, ws_need);
+    }
+    if (hd == 64) {
+        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, zero, part_bytes, st, ws_need);
+        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, zero, part_bytes, st, ws_need);
+        return launch_bwd<64, 4, 1>(a, vr, zero, part_bytes, st, ws_need);
+    }
+    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, zero, part_bytes, st, ws_need);
+    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, zero, part_bytes, st, ws_need);
+    return launch_bwd<32, 4, 2>(a, vr, zero, part_bytes, st, ws_need);
+}
+
 extern "C" int64_t mb_flash_ema_bwd_workspace(int hd, int N) {
     if (hd < 1 || N < 1) return 0;
     return device_cus() * bwd_dw_bytes(hd, rate_tiles(N));
+}
+
+extern "C" int64_t mb_flash_ema_bwd_lists_workspace(int B, int H, int L, int hd, int K, int N, int flags) {
+    FlashArgsV a{};
+    a.B = B; a.H = H; a.L = L; a.hd = hd; a.K = K; a.N = N; a.Np = N; a.Br = 64;
+    a.nc = L > 0 ? (L + 63) / 64 : 1;
+    if (flash_validate("mb_flash_ema_bwd_lists_workspace", a, hd)) return -1;
+    if (B == 0 || L == 0) return 0;
+    int64_t need = 0;
+    if (bwd_dispatch(a, hd, N, flags, false, ZeroFill{}, 0, nullptr, &need)) return -1;
+    return need;
 }
 
 extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,
@@ -741,7 +794,6 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     MB_REQUIRE(workspace_bytes >= 0, "mb_flash_ema_bwd: negative workspace size %lld", (long long)workspace_bytes);
     MB_REQUIRE(((uintptr_t)workspace & 15) == 0, "mb_flash_ema_bwd: workspace must be 16-byte aligned");
     a.dWpart = static_cast<float*>(workspace);
-    const int64_t part_bytes = workspace ? workspace_bytes : 0;
     const bool vr = (flags & MB_FLASH_VOCAB_ROWS) != 0;
     a.e_rows = vr ? V_total : 0;
     int rc = flash_validate("mb_flash_ema_bwd", a, hd);
@@ -761,35 +813,7 @@ extern "C" int mb_flash_ema_bwd_lists(const float* Q, int64_t q_sb, int64_t q_sh
     MB_REQUIRE(Q && dO && x && rhos && unique && O && LSE && W_pe && dQ,
                "mb_flash_ema_bwd: null pointer");
     MB_REQUIRE(K == 0 || (E_k && E_v && C_bounds), "mb_flash_ema_bwd: null slot pointer");
-    const int NS = rate_tiles(N);
-    const int gm = flash_gate_mode("mb_flash_ema_bwd", flags, N, hd);
-    if (gm < 0) return gm;
-    if (gm == 2) {
-        // hi + lo tiles of both kinds and both W fragment sets in LDS: one slot per batch at
-        // head_dim 64, two (N > 32) or four at head_dim 32, whose W fragments and rows take half:
-        // a batch's barrier, loads and stores are shared by its slots, and a slot of 32 dims is
-        // too short to cover them (B3 T201 H6 N33: backward 449 us with one slot per batch, 356 us
-        // with two).
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 1, true, true>(a, vr, zero, part_bytes, st) : launch_bwd<64, 2, 1, true, true>(a, vr, zero, part_bytes, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true, true>(a, vr, zero, part_bytes, st) : launch_bwd<32, 2, 2, true, true>(a, vr, zero, part_bytes, st);
-    }
-    if (gm == 1) {  // the gate's lo tile and W_lo beside the hi ones
-        if (hd == 64) return NS == 1 ? launch_bwd<64, 1, 4, true>(a, vr, zero, part_bytes, st) : launch_bwd<64, 2, 2, true>(a, vr, zero, part_bytes, st);
-        return NS == 1 ? launch_bwd<32, 1, 4, true>(a, vr, zero, part_bytes, st) : launch_bwd<32, 2, 2, true>(a, vr, zero, part_bytes, st);
-    }
-    if (hd == 128) {  // two 64-dim sub-heads per head
-        if (NS == 1) return launch_bwd<64, 1, 4, false, false, true>(a, vr, zero, part_bytes, st);
-        if (NS == 2) return launch_bwd<64, 2, 4, false, false, true>(a, vr, zero, part_bytes, st);
-        return launch_bwd<64, 4, 1, false, false, true>(a, vr, zero, part_bytes, st);
-    }
-    if (hd == 64) {
-        if (NS == 1) return launch_bwd<64, 1, 4>(a, vr, zero, part_bytes, st);
-        if (NS == 2) return launch_bwd<64, 2, 4>(a, vr, zero, part_bytes, st);
-        return launch_bwd<64, 4, 1>(a, vr, zero, part_bytes, st);
-    }
-    if (NS == 1) return launch_bwd<32, 1, 4>(a, vr, zero, part_bytes, st);
-    if (NS == 2) return launch_bwd<32, 2, 4>(a, vr, zero, part_bytes, st);
-    return launch_bwd<32, 4, 2>(a, vr, zero, part_bytes, st);
+    return bwd_dispatch(a, hd, N, flags, vr, zero, workspace ? workspace_bytes : 0, st, nullptr);
 }
 
 extern "C" int mb_flash_ema_bwd(const float* Q, int64_t q_sb, int64_t q_sh, int64_t q_sl,

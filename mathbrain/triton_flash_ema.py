@@ -282,6 +282,14 @@ def _fwd_workspace_bytes(B, H, L, hd, K, N, flags, device_index):
     return int(n)
 
 
+@functools.lru_cache(maxsize=256)
+def _bwd_workspace_bytes(B, H, L, hd, K, N, prec, device_index):
+    """Bytes of the backward's dW_pe workspace (mb_flash_ema_bwd_lists_workspace: 0 for a grid that
+    adds with atomics) on the current device, which is `device_index`; 0 for shapes that the
+    backward refuses, whose call raises."""
+    return max(0, int(_lib.lib().mb_flash_ema_bwd_lists_workspace(B, H, L, hd, K, N, prec)))
+
+
 def _fwd_fake(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, V_total, use_silu, Br, absent_mass,
               prec):
     B, H, L, hd = Q.shape
@@ -397,8 +405,8 @@ def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V
     with torch.cuda.device(dev):
         if lists is None:
             lists = _slot_lists(xl, uniq, Cb, N, Br)
-        nws = int(_lib.lib().mb_flash_ema_bwd_workspace(hd, N))
-        ws = torch.empty(nws, dtype=torch.uint8, device=dev)
+        nws = _bwd_workspace_bytes(B, H, L, hd, K, N, prec, dev.index)
+        ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
         _lib.call("mb_flash_ema_bwd_lists", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(dOf), _lib.ptr(xl),
                   xl.stride(0), xl.stride(1), _lib.ptr(Ek), _lib.ptr(Ev), _lib.ptr(W),
                   _lib.ptr(rh), _lib.ptr(uniq), _lib.ptr(Cb), _lib.ptr(Of), _lib.ptr(Lf), B, H, L,

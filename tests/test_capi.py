@@ -110,6 +110,26 @@ def test_backward_workspace_holds_every_workgroup(lib, hd):
         assert _lib.lib().mb_flash_ema_bwd_workspace(hd, N) >= 256 * a_workgroup, N
 
 
+def test_backward_workspace_is_asked_for_where_it_is_used(lib):
+    """mb_flash_ema_bwd_lists_workspace: the dW_pe sums of a grid that runs at once (at most 256
+    workgroups), never more than mb_flash_ema_bwd_workspace; nothing for a larger grid, which adds
+    with atomics, nor from the backward's Python entry point there."""
+    from mathbrain import _lib
+    from mathbrain.triton_flash_ema import _bwd_workspace_bytes
+    size = lambda *shape: _lib.lib().mb_flash_ema_bwd_lists_workspace(*shape, 0)  # noqa: E731
+    assert size(56, 8, 512, 64, 1638, 64) == 0 and size(16, 8, 4096, 64, 3900, 128) == 0
+    assert _bwd_workspace_bytes(56, 8, 512, 64, 1638, 64, 0, 0) == 0
+    assert size(0, 8, 512, 64, 1638, 64) == 0 and size(1, 8, 0, 64, 1638, 64) == 0
+    assert size(1, 8, 64, 48, 10, 16) == -1                                        # head_dim 48
+    # 8 groups of 64 batches of two slots in 32 parts: 256 workgroups of 4 x 32 columns, 128 rates
+    assert size(2, 4, 128, 32, 128, 80) == 256 * 4 * 32 * 128 * 4
+    assert size(1, 4, 32, 32, 0, 16) == 1 * 4 * 32 * 32 * 4                        # no slots: one part
+    for hd in (32, 64, 128):
+        for N in (1, 32, 33, 64, 65, 96, 97, 128):
+            for B, L, K in ((1, 1, 1), (2, 128, 400), (8, 512, 300), (3, 201, 5000)):
+                assert 0 <= size(B, 4, L, hd, K, N) <= _lib.lib().mb_flash_ema_bwd_workspace(hd, N)
+
+
 @pytest.mark.parametrize("K", [60, 150, 979, 1638])
 def test_forward_parts_fit_the_rounds(lib, K):
     """The forward's slot parts (read from its workspace: parts x rows x (hd + 2) floats) on grids
