@@ -218,11 +218,12 @@ def _slot_rows(E, B, K, D, V_total, what):
 MIN_LISTED_SLOTS = 16384
 
 
-def _slot_lists(xl, uniq, Cb, N, Br):
-    """The blocks' slot lists of mb_flash_ema_slot_lists (None for a call too small for them)."""
+def _slot_lists(xl, uniq, Cb, N, Br, always=False):
+    """The blocks' slot lists of mb_flash_ema_slot_lists (None for a call too small for them,
+    unless ``always``)."""
     B, L = xl.shape
     K = uniq.shape[1]
-    if B * -(-L // 32) * K < MIN_LISTED_SLOTS:
+    if not always and B * -(-L // 32) * K < MIN_LISTED_SLOTS:
         return None
     nbytes = _lib.lib().mb_flash_ema_slot_lists_bytes(B, L, K)
     lists = torch.empty(nbytes, dtype=torch.uint8, device=xl.device)
@@ -371,7 +372,9 @@ def _forward_with_scores(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, uniq
 
 
 def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V_total, use_silu,
-              Br, absent_mass, scores, prec=0, lists=None):
+              Br, absent_mass, scores, prec=0, lists=None, listed=False):
+    """``lists``: the forward's slot lists; ``listed``: it walked such lists, so that ``scores`` hold
+    only what they name (made again if ``lists`` is None)."""
     dev = _lib.require_gpu(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO,
                            what="flash_ema_backward")
     check_counter_range(rhos, "flash_ema_backward")
@@ -404,7 +407,7 @@ def _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE, dO, V
         raise ValueError(f"scores must be contiguous fp32 [B, H, K_max, L], got {tuple(scores.shape)}")
     with torch.cuda.device(dev):
         if lists is None:
-            lists = _slot_lists(xl, uniq, Cb, N, Br)
+            lists = _slot_lists(xl, uniq, Cb, N, Br, always=listed)
         nws = _bwd_workspace_bytes(B, H, L, hd, K, N, prec, dev.index)
         ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
         _lib.call("mb_flash_ema_bwd_lists", _lib.ptr(Qf), *Qf.stride(), _lib.ptr(dOf), _lib.ptr(xl),
@@ -463,9 +466,10 @@ def flash_ema_backward(Q, x, E_k, E_v, W_pe, rhos, V_total, unique_tensor, C_bou
 # 21.05 ms (no score products and half the cross-lane sums), 31.6 -> 30.5 ms per layer.
 # SAVE_SCORES_MAX_BYTES is a budget per device shared by every saved score tensor still
 # alive (a model's layers each keep theirs until the backward reaches them): a call whose
-# scores would take the held total past it recomputes them in the backward instead.  A
-# saved tensor returns its bytes when it is freed (after the backward, or when the graph is
-# dropped).  Traced graphs never save them.
+# scores would take the held total past it recomputes them in the backward instead.  The slot
+# lists kept with the scores (1 / (8 H) of their bytes) count too: where they no longer fit, the
+# backward lists the slots again.  A saved tensor returns its bytes when it is freed (after the
+# backward, or when the graph is dropped).  Traced graphs never save them.
 SAVE_SCORES = True
 SAVE_SCORES_MAX_BYTES = 16 << 30
 
@@ -522,6 +526,15 @@ def _reserve_scores(Q, K_max):
     return nbytes if score_budget.reserve(Q.device, nbytes, SAVE_SCORES_MAX_BYTES) else 0
 
 
+def _keep_lists(lists):
+    """``lists`` if their bytes fit the shared budget, which they hold until they are freed; else
+    None."""
+    if lists is None or not score_budget.reserve(lists.device, lists.numel(), SAVE_SCORES_MAX_BYTES):
+        return None
+    score_budget.hold(lists, lists.numel())
+    return lists
+
+
 class FlashEMAFunction(torch.autograd.Function):
     """Autograd entry point with the reference's 12 arguments (triton_flash_ema.py:571-650)
     and two more: apply(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_tensor,
@@ -555,7 +568,8 @@ class FlashEMAFunction(torch.autograd.Function):
             score_budget.hold(res[5], nbytes)
         O, LSE, C_bounds, E_k, E_v = res[:5]
         ctx.save_for_backward(Q, x, E_k, E_v, W_pe, rhos, C_bounds, unique_tensor, O, LSE,
-                              res[5] if keep else None, res[6] if keep else None)
+                              res[5] if keep else None, _keep_lists(res[6]) if keep else None)
+        ctx.listed = keep and res[6] is not None
         ctx.V_total = V_total
         ctx.use_silu = use_silu
         ctx.Br = Br
@@ -575,7 +589,7 @@ class FlashEMAFunction(torch.autograd.Function):
         else:
             dQ, dEk, dEv, dW = _bwd_impl(Q, x, E_k, E_v, W_pe, rhos, unique_tensor, C_bounds, O, LSE,
                                          dO.contiguous(), ctx.V_total, ctx.use_silu, ctx.Br, ctx.absent_mass,
-                                         S2, _prec(ctx.precision), lists)
+                                         S2, _prec(ctx.precision), lists, ctx.listed)
         if ctx.W_rows > dW.shape[0]:  # W_pe passed with padded rows: their gradient is 0
             dW = torch.cat([dW, dW.new_zeros(ctx.W_rows - dW.shape[0], dW.shape[1])])
         return dQ, None, dEk, dEv, dW, None, None, None, None, None, None, None, None, None

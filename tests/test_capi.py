@@ -199,6 +199,25 @@ def test_score_budget_is_shared_by_the_tensors_still_alive(monkeypatch):
     assert tfe._reserve_scores(Q, 1638) == 0
 
 
+def test_kept_slot_lists_count_in_the_score_budget(monkeypatch):
+    """The slot lists that a layer keeps beside its scores take their bytes from the same budget, are
+    not kept where they do not fit, and give the bytes back when freed."""
+    import gc
+    import torch
+    from mathbrain import triton_flash_ema as tfe
+    budget = tfe.ScoreBudget()
+    monkeypatch.setattr(tfe, "score_budget", budget)
+    monkeypatch.setattr(tfe, "SAVE_SCORES_MAX_BYTES", 1000)
+    assert tfe._keep_lists(None) is None
+    first = torch.empty(600, dtype=torch.uint8)
+    assert tfe._keep_lists(first) is first and budget.held("cpu") == 600
+    assert tfe._keep_lists(torch.empty(401, dtype=torch.uint8)) is None and budget.held("cpu") == 600
+    assert tfe._keep_lists(torch.empty(400, dtype=torch.uint8)) is not None
+    del first
+    gc.collect()
+    assert budget.held("cpu") == 0
+
+
 def test_counter_range_check_names_the_half_life_limit():
     """Rates whose key counters could leave the gate operands' fp16 range are refused on the
     host: the model with train.py's --max_hl 100000 raises at construction, and the

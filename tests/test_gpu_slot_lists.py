@@ -101,3 +101,34 @@ def test_lists_and_the_attention_over_them(L, N, Br, warmup, pad_slots, absent_m
                 continue
             assert torch.isfinite(a).all()
             assert norm_err(a, w) < (TOL_DW[prec] if i in (5, 9) else TOL)
+
+
+def autograd_grads(c, dO, precision="bf16"):
+    """O and the gradients of FlashEMAFunction."""
+    from mathbrain.triton_flash_ema import FlashEMAFunction
+    leaves = [t.cuda().requires_grad_(True) for t in (c["Q"], c["E_k"], c["E_v"], c["W"])]
+    O = FlashEMAFunction.apply(leaves[0], c["x"].cuda(), leaves[1], leaves[2], leaves[3], c["rhos"].cuda(), c["V"],
+                               c["unique"].cuda(), c["K"], c["Cb"].cuda(), True, c["Br"], True, precision)
+    return [t.cpu() for t in (O.detach(), *torch.autograd.grad(O, leaves, dO.cuda()))]
+
+
+def test_lists_beyond_the_score_budget_are_made_again(monkeypatch):
+    """With room for the scores and not for the lists, the backward lists the slots again, also where
+    the rule for small calls would now say otherwise: the gradients stay finite (the scores of pairs
+    outside the lists are never written) and are those with the lists kept."""
+    from mathbrain import triton_flash_ema as tfe
+    monkeypatch.setattr(tfe, "score_budget", tfe.ScoreBudget())
+    monkeypatch.setattr(tfe, "MIN_LISTED_SLOTS", 0)
+    c = make_case(2, 97, 700, 4, 32, 16, seed=4, qs=0.5, es=0.3, ws=0.2)
+    dO = torch.randn(c["Q"].shape, generator=torch.Generator().manual_seed(3))
+    want = autograd_grads(c, dO, "fp32")
+    monkeypatch.setattr(tfe, "SAVE_SCORES_MAX_BYTES", 4 * 2 * 4 * c["K"] * 97)
+    made = []
+    real = tfe._slot_lists
+    monkeypatch.setattr(tfe, "_slot_lists", lambda *a, **k: made.append(real(*a, **k)) or made[-1])
+    junk = torch.full((4 * 2 * 4 * c["K"] * 97,), 255, dtype=torch.uint8, device="cuda")  # NaN where the scores go
+    del junk
+    got = autograd_grads(c, dO, "fp32")
+    assert len(made) == 2 and all(m is not None for m in made)
+    for i, (a, w) in enumerate(zip(got, want)):
+        assert torch.isfinite(a).all() and norm_err(a, w) < (TOL_DW["fp32"] if i == 4 else TOL)
