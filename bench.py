@@ -11,8 +11,10 @@ dO N(0, 1) (synthetic, seeded).  One step = key-side chunk states (mb_ema_bounda
 Prints one JSON line.  `roofline` is for the dominant kernel (the backward): algorithmic
 flops per launch, sum_b L*K_b*(4*N*D + 10*D) (gate recompute, dW_pe and five
 per-element products: dO . (e_v g), dQ, dE_k, dE_v and dpre; the scores come from the
-forward, as FlashEMAFunction keeps them; only valid (t, k) pairs count), over its mean launch
+forward, as FlashEMAFunction keeps them; only the (t, k) pairs that the blocks' slot lists name
+count, which is what the kernels compute: the other valid pairs are zero), over its mean launch
 time measured with HIP events on the launch stream, against the dense bf16/fp16 MFMA peak of 2516.6 TFLOP/s.
+`config.listed_pairs` is those pairs' share of the valid ones.
 `cpu_baseline` times the CPU restatement of the reference algorithm (the oracle, a port
 of the reference's PyTorch path) on a bounded slice of the same workload on this host.
 
@@ -127,10 +129,10 @@ def attention_case(seed=0, config="cfg2"):
 
 
 def attention_step(c, timers=None, precision="bf16"):
-    from mathbrain.triton_flash_ema import (_forward_with_scores, _prec, flash_ema_backward,
+    from mathbrain.triton_flash_ema import (_bwd_impl, _forward_with_scores, _prec, flash_ema_backward,
                                             flash_ema_forward, keep_scores, precompute_boundaries)
-    # the forward keeps its scores for the backward when FlashEMAFunction would (the same
-    # call FlashEMAFunction makes then)
+    # the forward keeps its scores and slot lists for the backward when FlashEMAFunction would
+    # (the same calls FlashEMAFunction makes then)
     keep = keep_scores(c["B"], c["H"], c["K"], c["L"])
     Cb = precompute_boundaries(c["x"], c["unique"], c["rhos"], 64, c["c_base"])
     if timers is not None:
@@ -145,12 +147,27 @@ def attention_step(c, timers=None, precision="bf16"):
     if timers is not None:
         timers["fwd"][1].record()
         timers["bwd"][0].record()
-    grads = flash_ema_backward(c["Q"], c["x"], c["E_k"], c["E_v"], c["W"], c["rhos"], c["V"],
-                               c["unique"], Cb, O, LSE, c["dO"], precision=precision,
-                               scores=res[5] if keep else None)
+    if keep:
+        grads = _bwd_impl(c["Q"], c["x"], c["E_k"], c["E_v"], c["W"], c["rhos"], c["unique"], Cb, O, LSE, c["dO"],
+                          c["V"], True, 64, True, res[5], _prec(precision), res[6], res[6] is not None)
+    else:
+        grads = flash_ema_backward(c["Q"], c["x"], c["E_k"], c["E_v"], c["W"], c["rhos"], c["V"],
+                                   c["unique"], Cb, O, LSE, c["dO"], precision=precision)
     if timers is not None:
         timers["bwd"][1].record()
     return grads
+
+
+def listed_pairs(c):
+    """(step, slot) pairs that the blocks' slot lists of the case name, which both kernels walk."""
+    from mathbrain.triton_flash_ema import _slot_lists, precompute_boundaries
+    B, L, K = c["B"], c["L"], c["K"]
+    Cb = precompute_boundaries(c["x"], c["unique"], c["rhos"], 64, c["c_base"])
+    lists = _slot_lists(c["x"], c["unique"], Cb, c["N"], 64, always=True)
+    blocks = -(-L // 32)
+    counts = lists[16 * B * blocks * K:][:8 * B * blocks].view(torch.int32).view(B, blocks, 2)[..., 0]
+    steps = torch.tensor([min(32, L - 32 * i) for i in range(blocks)], device=counts.device)
+    return int((counts.long() * steps).sum())
 
 
 def cpu_baseline_attention(c, seconds=12.0):
@@ -235,7 +252,8 @@ def run_attention(args):
     fwd_ms = sum(t["fwd"][0].elapsed_time(t["fwd"][1]) for t in timers_all) / args.steps
     bwd_ms = sum(t["bwd"][0].elapsed_time(t["bwd"][1]) for t in timers_all) / args.steps
     L, N, D = c["L"], c["N"], c["D"]
-    pairs = int(c["counts"].sum()) * L          # valid (t, k) pairs
+    valid_pairs = int(c["counts"].sum()) * L    # of the sequences' own slots
+    pairs = listed_pairs(c)                     # those that the kernels walk
     fwd_flop = pairs * (2 * N * D + 4 * D)
     bwd_flop = pairs * (4 * N * D + 10 * D)
     tokens = c["B"] * L
@@ -263,6 +281,7 @@ def run_attention(args):
         "config": {"workload": workload,
                    "B": c["B"], "T": L, "d_model": D, "heads": c["H"], "head_dim": c["hd"],
                    "N": N, "V": c["V"], "K_max": c["K"], "sum_K_b": int(c["counts"].sum()),
+                   "listed_pairs": round(pairs / valid_pairs, 4),
                    "fwd_ms": round(fwd_ms, 4), "bwd_ms": round(bwd_ms, 4),
                    "fwd_bwd_tflops": round((fwd_flop + bwd_flop) / ((fwd_ms + bwd_ms) * 1e-3) / 1e12, 2),
                    "precision": args.precision, "parallelism": "single GPU"},
