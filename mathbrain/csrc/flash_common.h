@@ -1,7 +1,8 @@
 // Pieces shared by the flash-EMA forward and backward kernels (gfx950).
 //
 // Both kernels work on one (sequence b, 32-step block) per workgroup and walk the block's
-// slots (its list, flash_slots.hip, or all valid slots of b) in batches of SB.  For every batch the whole workgroup first builds, in LDS,
+// slots (its list, flash_slots.hip, or all valid slots of b) in batches of SB.  For every batch the
+// whole workgroup first builds, in LDS,
 //   cdec[j][t][n]  (fp16)  the decayed key-side counter c_dec[t, u_j, n] that gates step t,
 //   cdecT[j][n][t] (bf16)  the same counter, transposed, for the backward's dW_pe product,
 //   E[j][0|1][D]   (fp32)  the slot's key and value embeddings,
@@ -140,6 +141,8 @@ inline int device_cus() {
 // parts; beyond that the rounds even out by themselves.  Measured, backward + forward kernels:
 // B3 T201 H6 N33 in fp32 mode 356 + 96 -> 81 + 49 us; B2 T128 H4 N16 83 + 32 -> 27 + 24 us;
 // B8 T512 H8 of documents (0.5 and 1 rounds) two parts 2.57 + 2.57 ms, four 2.35 + 1.37 ms.
+// Lists that are all equally long have nothing to even out and pay for it: B8 T512 H8 with every
+// slot active, backward 3.20 -> 3.33 ms, forward 1.63 -> 1.66.
 constexpr int kPartsMax = 32;
 constexpr int kPartBatches = 32;
 inline int slot_parts(int64_t G, int64_t conc, int nbatch) {
@@ -250,7 +253,8 @@ __device__ inline float row_sum16(float v) {
 // XCDs round-robin): given sequences of its own, whose slot embeddings would share its L2, an XCD
 // with short lists waits for one with long ones (B8 T512 of documents: backward 5.05 -> 3.37 ms,
 // forward 2.69 -> 1.84), and sharing did not pay where they are equally long either (B56 T512
-// 20.6 -> 20.5 ms without).
+// 20.6 -> 20.5 ms without): the rows then come from memory more often (forward 0.6 -> 4.9 GB,
+// 0.46 TB/s, backward 2.2 -> 6.6 GB), which bounds neither kernel.
 struct FlashBlock {
     int b, t, r;
 };
@@ -335,8 +339,9 @@ __device__ void flash_powers(const FlashArgs& a, float* powt) {
         powt[j * NPAD + n] = n < a.N ? pow_steps(hi, lo, j) : 0.0f;
 }
 
-// Per-block setup shared by both kernels: the match window tokens, kinfo[0] = the valid slots of sequence b and kinfo[1] = the slots to walk (the
-// length of the block's list, or without lists one past the last valid slot).
+// Per-block setup shared by both kernels: the match window tokens, kinfo[0] = the valid slots of
+// sequence b and kinfo[1] = the slots to walk (the length of the block's list, or without lists one
+// past the last valid slot).
 __device__ inline void flash_setup(const FlashArgs& a, int b, int t0, int cb, int64_t* win, int* kinfo) {
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;

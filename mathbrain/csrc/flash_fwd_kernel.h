@@ -434,12 +434,12 @@ flash_fwd_merge_kernel(const float* __restrict__ part, int ks, int64_t rows, flo
 // slot_parts, which even out lists of different lengths, or up to four more where that shortens
 // equally long ones by at least 7.5 %: rounds x (batches of a part + kPartPrice, what a part
 // repeats).  448 workgroups at B28 T512 H8 N64 take 6 rounds of 256 in slot_parts' three parts
-// (2.0 of a whole walk), 7 in four (1.75): 6.45 -> 5.73 ms; 288 with 150 slots take two rounds whole, 5 in
-// four parts: 654 -> 527 us.  Batches of documents pay up to 7 % for it (B11 0.94 -> 1.00 ms); fewer
+// (2.0 of a whole walk), 7 in four (1.75): 6.45 -> 5.73 ms; 288 with 150 slots take two rounds
+// whole, 5 in four parts: 654 -> 527 us.  Batches of documents pay up to 7 % for it (B11 0.94 -> 1.00 ms); fewer
 // parts than slot_parts' would cost them more (four for seven: 1.32 ms).
 // From two rounds on the workgroups of equally long lists end their rounds together, and a split
 // must save at least 3 % of them: 896 at B56 T512 take 4 where 3.5 would do (two parts: 10.22 ->
-// 9.12 ms with single products).  Every part keeps four batches.
+// 9.12 ms with single products).  What is split beyond slot_parts' parts keeps four batches a part.
 constexpr double kPartPrice = 4.0;
 static int fwd_parts(int64_t G, int64_t conc, int nbatch) {
     if (G <= 0 || conc <= 0) return 1;

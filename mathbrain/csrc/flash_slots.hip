@@ -12,8 +12,11 @@
 // N128 backward 107.1 -> 83.7 ms and forward 38.5 -> 33.0 ms; B56 T512 N64 21.6 -> 20.1 and
 // 10.8 -> 10.7 ms; a forward over one 10 001-step sequence 7.78 -> 5.31 ms.
 //
-// Bound: one read of C_bounds (1.27 GB at B16 T4096 N128, 0.50 ms; 183 MB at B56 T512, 70 us)
-// in rows of N floats by whole waves; the lists and the unique ids are under a tenth of it.
+// Bound: the read of C_bounds in rows of N floats by whole waves.  Per slot and chunk of 64 steps
+// 4 N bytes and 8 of the id are read and up to 32 written (two entries): the rest is a sixth of
+// the rows at N = 64, a twelfth at 128 and over half at 16.  B56 T512 N64 216 MB in 70 us, B16
+// T4096 N128 1.36 GB in 454 us (3.0 TB/s both); a grid of few (sequence, chunk) pairs is bound by
+// the latency of a workgroup's rounds of 512 slots instead (B8 T512, 64 workgroups: 41 us).
 #include "flash_common.h"
 
 namespace mb {

@@ -30,7 +30,8 @@ def flash_ema_forward(Q, x, E_k_slots, E_v_slots, rhos, pe_proj, n_heads, use_si
     hd = D // H
     unique, K_max = _build_unique_index(x, Q.device)
     # index_select: its backward adds the rows' gradients in one launch, an index's sorts them
-    # first (forward and backward at B2 L128 H4 head_dim 32: 35 launches and 597 us, now 22 and 331)
+    # first (forward and backward at B2 L128 H4 head_dim 32: 35 launches, now 21; the call, with
+    # the attention's slot parts, 564 -> 518 us, the host's time)
     rows = unique.clamp(min=0).view(-1)
     E_k = E_k_slots.index_select(0, rows).view(B, K_max, *E_k_slots.shape[1:])
     E_v = E_v_slots.index_select(0, rows).view(B, K_max, *E_v_slots.shape[1:])

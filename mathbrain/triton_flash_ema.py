@@ -211,10 +211,12 @@ def _slot_rows(E, B, K, D, V_total, what):
     return Ef.contiguous(), False
 
 
-# Blocks x slots below which a call walks every slot instead of listing the active ones: the
-# lists cost a launch of 10 to 30 us, and a call this small spends no more than that on the
-# slots they leave out (B3 T201 N33 in fp32 mode, about 9 000: 577 us without, 616 us with; B8
-# T512, 96 000: 17.6 ms for a 2-layer model's step either way; above that the lists win).
+# Blocks x slots below which a call walks every slot instead of listing the active ones.  The
+# lists cost two launches, 50 us at B8 T512 and 75 at B56 T512, which a training step repays where
+# they leave slots out.  Time of forward and backward over every slot : over lists, with a history
+# of 300 to 4 096 tokens (and without one): up to 13 000 blocks x slots 0.95-0.97 (0.91-0.97),
+# 17 000 to 26 000 0.96-1.00 (0.99-1.24), 36 000 to 54 000 1.01-1.09 (1.35), from 93 000 up
+# 1.04-1.15.  A forward alone gains later: 0.77-0.90, 0.83-1.03 (0.94-1.36) and 1.02-1.08.
 MIN_LISTED_SLOTS = 16384
 
 
@@ -334,6 +336,9 @@ def flash_ema_forward(Q, x, E_k_active, E_v_active, W_pe, rhos, V_total, unique_
     operands into fp16 hi + lo pairs (N <= 64, head_dim <= 64; single fp16 operands
     beyond), "fp16" takes single fp16 operands (faster; for small scores only), "fp32" also
     splits the backward's dW_pe product.
+    Calls of MIN_LISTED_SLOTS blocks x slots or more, without ``return_scores``, walk per block of 32
+    steps only the slots whose counters can be nonzero in it: a non-finite E_k / E_v row does not
+    reach the blocks that leave its slot out (walked over, 0 times it would be NaN there too).
     """
     prec = _prec(precision)
     B, H, L, hd = Q.shape
@@ -450,7 +455,9 @@ def flash_ema_backward(Q, x, E_k, E_v, W_pe, rhos, V_total, unique_tensor, C_bou
     ``scores`` is the forward's optional scores output (recomputed when None).  Returns
     (dQ [B,H,L,hd], dE_k [B,K,H*hd], dE_v [B,K,H*hd], dW_pe [N, H*hd]), all fp32.
     ``precision`` as in flash_ema_forward ("fp32" also takes the dW_pe product from bf16
-    hi + lo pairs of both operands).
+    hi + lo pairs of both operands).  dE_k, dE_v and dW_pe add with atomics, and so does dQ where a
+    grid below two rounds of workgroups splits its slots into parts: their last bits can differ
+    from call to call.
     """
     prec = _prec(precision)
     if scores is None:
